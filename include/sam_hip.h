@@ -56,8 +56,9 @@ int sam_hip_enabled(void);
  * hd <= 128. Which kernel runs (f16/bf16) is chosen for speed only; every shape within the limits gets
  * the same result to the same tolerance. Dedicated kernels take SAM's two shapes at hd 64 and 80:
  * windows with 13 <= h <= 16 and an even w <= 16, and the 64-column global grid (w == 64, h <= 64) when
- * 2^-6 <= scale * log2(e) <= 4 (SAM's hd^-0.5 * log2(e) is 0.16-0.18). Every other shape or scale up to
- * 64 x 64 runs on the general kernel, and grids past 64 rows or columns on a kernel that walks them in
+ * 2^-6 <= scale * log2(e) <= 4 (SAM's hd^-0.5 * log2(e) is 0.16-0.18). Other grids up to 64 x 64 at those
+ * head dims and scales run on a kernel that packs the grid rows into tiles (except some whose width is 25..32
+ * or 57..64). Every other shape or scale up to 64 x 64 runs on the general kernel, and grids past 64 rows or columns on a kernel that walks them in
  * 64-column passes, each at a lower speed. The reference's own GPU sequence stops at h*w <= 8192 (the
  * relpos_softmax row limit); here the scores stay on chip, so every h, w <= 128 runs. In f32, hd 64 has
  * its own window kernel (w <= 16, h <= 16, h*w <= 256) and global kernel (w == 64); other f32 shapes run

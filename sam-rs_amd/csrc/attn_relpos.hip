@@ -540,6 +540,9 @@ bool attn_relpos_window(int dtype, const void* q, const void* kt, const void* v,
 bool attn_relpos_global(int dtype, const void* q, const void* kt, const void* v, const void* table, void* out, int bh,
                         int hd, int h, int w, float scale, hipStream_t stream, hipError_t* err);
 
+bool attn_relpos_rows(int dtype, const void* q, const void* kt, const void* v, const void* table, void* out, int bh,
+                      int hd, int h, int w, float scale, hipStream_t stream, hipError_t* err);
+
 hipError_t attn_relpos_wide(int dtype, const void* q, const void* kt, const void* v, const void* table, void* out,
                             int bh, int hd, int h, int w, float scale, hipStream_t stream);
 
@@ -549,9 +552,11 @@ hipError_t attn_relpos_half(int dtype, const void* q, const void* kt, const void
   // grids past 64 rows or columns (up to 128): attn_relpos_wide.hip
   if (h > 64 || w > 64) return attn_relpos_wide(dtype, q, kt, v, table, out, bh, hd, h, w, scale, stream);
   // windowed grids (the 14x14 SAM windows): attn_relpos_win.hip; the 64-column global grid:
-  // attn_relpos_glob.hip; every other shape: the general kernel below
+  // attn_relpos_glob.hip; other grids at hd 64 and 80: attn_relpos_rows.hip; every other shape: the general
+  // kernel below
   if (attn_relpos_window(dtype, q, kt, v, table, out, bh, hd, h, w, scale, stream, &e)) return e;
   if (attn_relpos_global(dtype, q, kt, v, table, out, bh, hd, h, w, scale, stream, &e)) return e;
+  if (attn_relpos_rows(dtype, q, kt, v, table, out, bh, hd, h, w, scale, stream, &e)) return e;
   if (dtype == kF16) return pick_hd<f16>(q, kt, v, table, out, bh, hd, h, w, scale, stream);
   return pick_hd<bf16>(q, kt, v, table, out, bh, hd, h, w, scale, stream);
 }

@@ -1,0 +1,45 @@
+"""Parity of the packed-row rel-pos kernel (attn_relpos_rows.hip, f16 / bf16 grids of any width at hd 64 and
+80) with the CPU oracle, on an MI355X, at the sizes where its tiling can go wrong."""
+import pytest
+import torch
+
+import sam_oracle as oracle
+from parity import check
+from test_attn_relpos_gpu import hip, make_inputs, run_gpu  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# Every chunk count per row (1..8) with full, one-column and odd last chunks; grids of less than a tile and
+# of one token; tiles that end inside a row and exactly on one; 128 and 129 tokens (the line between one
+# wave group and two) and odd row counts, whose halves differ; heights up to 64; and bh that gives one group
+# of 256 queries (300 heads of 9 x 17) and two.
+GRIDS = [(1, 1, 2), (1, 7, 2), (3, 5, 2), (8, 8, 2), (16, 8, 2), (43, 3, 2), (64, 1, 2), (9, 9, 2), (13, 13, 2),
+         (64, 16, 1), (5, 17, 2), (9, 17, 300), (16, 24, 2), (5, 25, 3), (10, 32, 2), (11, 33, 2), (24, 40, 1),
+         (7, 41, 2), (8, 48, 2), (9, 49, 2), (37, 50, 2), (8, 56, 2), (5, 57, 2), (3, 63, 2)]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("h,w,bh", GRIDS)
+def test_packed_rows_match_oracle(hip, h, w, bh, hd, dtype):  # noqa: F811
+    print(f"packed rows {dtype} {h}x{w} bh={bh} hd={hd}", flush=True)
+    arrays = make_inputs(h, w, bh, hd, 700 + 64 * h + w + hd, dtype, table_std=0.5)
+    scale = hd ** -0.5
+    got = run_gpu(hip, arrays, h, w, scale, dtype)
+    heads = [0, bh - 1]
+    q, kt, v, table = arrays
+    want = oracle.attention_relpos(q[heads], kt[heads], v[heads], table, h, w, scale)
+    check(got[heads], want, dtype, f"packed rows {h}x{w} hd={hd} {dtype}")
+
+
+@pytest.mark.parametrize("h,w", [(9, 13), (11, 33)])
+def test_packed_rows_keep_a_head_to_itself(hip, h, w):  # noqa: F811
+    """kT is read in 16-byte pieces that pass the end of a row; NaN keys and values in one head must not
+    reach its neighbours."""
+    bh, hd = 3, 64
+    q, kt, v, table = make_inputs(h, w, bh, hd, 5, "f16")
+    clean = run_gpu(hip, [q, kt, v, table], h, w, hd ** -0.5, "f16")
+    kt[1], v[1] = float("nan"), float("nan")
+    got = run_gpu(hip, [q, kt, v, table], h, w, hd ** -0.5, "f16")
+    assert (got[[0, 2]] == clean[[0, 2]]).all()
+    assert torch.from_numpy(got[1]).isnan().all()
