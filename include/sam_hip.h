@@ -60,9 +60,9 @@ int sam_hip_enabled(void);
  * head dims and scales run on a kernel that packs the grid rows into tiles (except some whose width is 25..32
  * or 57..64). Every other shape or scale up to 64 x 64 runs on the general kernel, and grids past 64 rows or columns on a kernel that walks them in
  * 64-column passes, each at a lower speed. The reference's own GPU sequence stops at h*w <= 8192 (the
- * relpos_softmax row limit); here the scores stay on chip, so every h, w <= 128 runs. In f32, hd 64 has
- * its own window kernel (w <= 16, h <= 16, h*w <= 256) and global kernel (w == 64); other f32 shapes run
- * on the general f32 kernel.
+ * relpos_softmax row limit); here the scores stay on chip, so every h, w <= 128 runs. In f32, hd 64 and
+ * 80 run on the bf16 matrix units with every operand as three bf16 terms (f32 products and sums), other head
+ * dims on the f32 matrix units.
  */
 int sam_hip_attn_relpos(const void* q, const void* kt, const void* v, const void* table, void* out, int dtype,
                         int bh, int h, int w, int hd, float scale, void* stream);

@@ -1,0 +1,64 @@
+"""Parity of the f32 rel-pos kernel on three bf16 terms (attn_relpos_f32_split.hip, hd 64 and 80) with the CPU
+oracle, on an MI355X, at the sizes where its tiling can go wrong."""
+import numpy as np
+import pytest
+
+import sam_oracle as oracle
+from parity import check
+from test_attn_relpos_gpu import hip, make_inputs, run_gpu  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# Every chunk count per row (1..8) with full, one-column and odd last chunks; grids of less than a tile of 32
+# slots and of one row; tables that fit in LDS whole (up to 28 rows and columns in all) and in several pieces;
+# odd row counts, whose halves differ; and bh that gives each of the three workgroups: two groups (few heads),
+# 4 waves (300 heads of 14 x 14) and 8 waves (12 heads of 60 x 60).
+GRIDS = [(1, 1, 2), (1, 7, 2), (1, 64, 2), (3, 5, 2), (8, 8, 2), (16, 8, 2), (43, 3, 2), (64, 1, 2), (9, 9, 2),
+         (13, 15, 2), (14, 14, 300), (64, 16, 1), (5, 17, 2), (16, 24, 2), (5, 25, 3), (10, 32, 2), (11, 33, 2),
+         (24, 40, 1), (7, 41, 2), (8, 48, 2), (37, 50, 2), (8, 56, 2), (5, 57, 2), (3, 63, 2), (60, 60, 12)]
+
+
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("h,w,bh", GRIDS)
+def test_f32_split_matches_oracle(hip, h, w, bh, hd):  # noqa: F811
+    print(f"f32 split {h}x{w} bh={bh} hd={hd}", flush=True)
+    # The oracle's own f32 sums are 9.8e-6 from 64 bits at 3600 keys with a table of deviation 0.5 (the kernel
+    # 1.3e-6), as much as the bar of 1e-5; with 0.02 the oracle is 3.5e-6 from them.
+    arrays = make_inputs(h, w, bh, hd, 900 + 64 * h + w + hd, "f32", table_std=0.02 if h * w > 2000 else 0.5)
+    scale = hd ** -0.5
+    got = run_gpu(hip, arrays, h, w, scale, "f32")
+    heads = [bh - 1] if h * w > 2000 else [0, bh - 1]
+    q, kt, v, table = arrays
+    want = oracle.attention_relpos(q[heads], kt[heads], v[heads], table, h, w, scale)
+    check(got[heads], want, "f32", f"f32 split {h}x{w} hd={hd}")
+
+
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("h,w", [(9, 13), (11, 33)])
+def test_f32_split_infinities(hip, h, w, hd):  # noqa: F811
+    """An infinite key gives its queries a score of -inf (weight 0) or +inf (a NaN row) by the sign of q, an
+    infinite value an infinite output, as f32 arithmetic has it; other heads are untouched."""
+    bh, key, dim = 3, w + 2, 5
+    q, kt, v, table = make_inputs(h, w, bh, hd, 6, "f32")
+    clean = run_gpu(hip, [q, kt, v, table], h, w, hd ** -0.5, "f32")
+    kt[0, dim, key] = np.inf
+    v[1, key, dim] = -np.inf
+    got = run_gpu(hip, [q, kt, v, table], h, w, hd ** -0.5, "f32")
+    masked = q[0, :, dim] < 0
+    assert masked.any() and not masked.all()
+    assert np.isnan(got[0][~masked]).all()
+    finite = kt[0].copy()
+    finite[dim, key] = 0
+    qs = q[0].astype(np.float64)
+    i, j = np.divmod(np.arange(h * w), w)
+    t = table.astype(np.float64)
+    bias = np.einsum("nd,nkd->nk", qs, t[i[:, None] - i[None] + h - 1] + t[2 * h - 1 + j[:, None] - j[None] + w - 1])
+    logits = qs @ finite.astype(np.float64) * hd ** -0.5 + bias
+    logits[:, key] = -np.inf
+    p = np.exp(logits - logits.max(1, keepdims=True))
+    want = (p / p.sum(1, keepdims=True)) @ v[0].astype(np.float64)
+    check(got[0][masked], want[masked].astype(np.float32), "f32", f"-inf scores {h}x{w} hd={hd}")
+    assert np.isneginf(got[1][:, dim]).all()
+    rest = [d for d in range(hd) if d != dim]
+    check(got[1][:, rest], clean[1][:, rest], "f32", f"-inf value {h}x{w} hd={hd}")
+    assert (got[2] == clean[2]).all()
