@@ -166,6 +166,24 @@ __device__ __forceinline__ bf16x8 pack8(const float* v, bf16x8*) {
   return r;
 }
 
+// 8 f32 values as hi + lo bf16 (round to nearest even, about 16 bits in all), two at a time on the packed
+// conversion: hi goes back to f32 by a shift and a mask (from single elements the compiler converts each
+// a second time).
+__device__ __forceinline__ void split_hi_lo(const float* v, bf16x8& hi, bf16x8& lo) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  u32x4 h, l;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float a = v[2 * i], b = v[2 * i + 1];
+    h[i] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
+    const float ra = a - __uint_as_float(h[i] << 16), rb = b - __uint_as_float(h[i] & 0xffff0000u);
+    l[i] = __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{ra, rb}, bf16x2));
+  }
+  hi = __builtin_bit_cast(bf16x8, h);
+  lo = __builtin_bit_cast(bf16x8, l);
+}
+
 __device__ __forceinline__ int wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
 
 }  // namespace samhip

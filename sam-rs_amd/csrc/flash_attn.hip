@@ -40,9 +40,12 @@ constexpr float kFlashLog2e = 1.4426950408889634f;
 template <typename T, int DP, int NW>
 struct FlashGeom {
   static constexpr int KS = DP / 16;        // k-steps of S^T = K Q^T
-  static constexpr int MBO = DP / 32;       // 32-row blocks of O^T
+  static constexpr int MBO = (DP + 31) / 32;  // 32-row blocks of O^T
+  static constexpr int PD = 32 * MBO;       // columns of a partial O row (flash_padded_dim)
   static constexpr int KSTR = DP + 8;       // K tile row stride (elements): rows 16 bytes apart mod 128
-  static constexpr int VSTR = DP + 16;      // V tile row stride: transpose reads shift 8 banks per row
+  // V tile row stride: 16 or 48 banks mod 64, so that the 4 rows x 32 columns of a half wave's transpose
+  // read fall on all 64 banks once (DP + 16 had two rows share 8 or 16 of them)
+  static constexpr int VSTR = 32 * MBO + (DP == 32 || MBO == 3 ? 0 : 32);
   static constexpr int KBUF = 64 * KSTR;
   static constexpr int VBUF = 64 * VSTR;
   static constexpr int NT = NW * 64;
@@ -66,14 +69,29 @@ __device__ __forceinline__ void rope_pair(float x0, float x1, float c0, float s0
   y1 = x1 * c1 + x0 * s1;
 }
 
+template <typename T, int DP, int NW, bool MASK>
+constexpr bool kThreePerSimd = NW == 4 && DP <= 64 && __is_same(T, f16) && !(DP == 64 && MASK);
+
 // f16 4-wave workgroups (head dims up to 64) are held to 168 registers, so that three share a CU (bf16,
-// whose P.V takes P as hi + lo, would spill there and runs two to a CU).
+// whose P.V takes P as hi + lo, would spill there and runs two to a CU). Up to head dim 128 the others are
+// held to 256 in all: without that bound the compiler keeps O in accumulation registers and copies it out
+// and back around the rescale.
+//
+// What bounds short key ranges (a window of 196 or 576 keys, 4 to 9 tiles) is the VALU's issue rate, beside
+// the first tiles' latency: a wave64 instruction takes 4 cycles, and a tile has 32 scores a lane. So the
+// staging keeps one 32-bit offset per chunk and a uniform base per tile, moves only the d columns that
+// exist (the pad is cleared once), and looks at the key range in the last tile alone; bf16 P is split on
+// packed conversions; a wave without queries only stages. 64 x 4 windows of 196 at head dim 72, bf16: 23.4 us
+// at 2613 VALU instructions a wave before, now 17.2 (f16 21.4 -> 14.6); 128 heads of 1024 at 96, f16 106.6 ->
+// 74.5; 144 of 576 at 64 28.9 -> 27.3 (bf16 36.2 -> 31.9); with a 196 x 196 bias, 320 heads at 32 31.1 -> 17.5.
 template <typename T, int DP, int NW, bool ROPEQ, bool MASK>
-__global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ? 3 : 1) void flash_fwd_kernel(
+__global__ __launch_bounds__(NW * 64, (kThreePerSimd<T, DP, NW, MASK> ? 3 : DP <= 128 ? 2 : 1)) void flash_fwd_kernel(
     FlashParams p) {
   typedef FlashGeom<T, DP, NW> FG;
   typedef typename Vec<T>::x8 X8;
   constexpr bool kSplitP = __is_same(T, bf16);
+  // at 168 registers there is no room for V(t+1) beside the scores; the other two waves cover its latency
+  constexpr bool kLateV = kThreePerSimd<T, DP, NW, MASK> && DP == 64;
   constexpr int KS = FG::KS, MBO = FG::MBO, KSTR = FG::KSTR, VSTR = FG::VSTR;
   constexpr int KBUF = FG::KBUF, VBUF = FG::VBUF, NT = FG::NT;
   constexpr int CPR = FG::CPR, CH = FG::CH, PT = FG::PT;
@@ -102,58 +120,73 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
   const int t_begin = split * p.tps;
   const int ntiles_all = (p.lk + 63) >> 6;
   const int t_end = min(ntiles_all, t_begin + p.tps);
-  const int ntiles = t_end - t_begin;
   const int kend = p.lk;  // keys >= kend are masked (only the last tile can hold such keys)
 
   const T* qbase = reinterpret_cast<const T*>(p.q) + bi * p.sq[0] + head * p.sq[2];
   const T* kbase = reinterpret_cast<const T*>(p.k) + bi * p.sk[0] + head * p.sk[2];
   const T* vbase = reinterpret_cast<const T*>(p.v) + bi * p.sv[0] + head * p.sv[2];
 
-  // ---- K/V tile staging: global -> registers -> LDS, zero outside [0, kend) x [0, d). Loads are
-  // unconditional (an out-of-range chunk reads the head's first row) so no branch sits between a
-  // load's issue and the work that hides its latency; the zero fill is applied at the LDS store.
+  // ---- K/V tile staging: global -> registers -> LDS, 16-byte chunks of the 64 x DP tile (loads of those
+  // past d read the row's last one and are not stored). A thread's chunks are the same (row, columns) in every tile, at 32-bit offsets from the
+  // tile's first row; where a round of threads covers whole rows (kStep) its next round is at a uniform
+  // distance. The last tile's rows past the end read the last key instead: its scores are masked, its V is
+  // stored as zeros. Row strides whose offsets do not fit in 32 bits take the path of the last tile.
+  constexpr bool kStep = NT % CPR == 0;
+  constexpr int RS = NT / CPR;  // rows of a round
+  const bool wide = max(p.sk[1], p.sv[1]) >= 1L << 24;
+  constexpr int NO = kStep ? 1 : PT;
+  int lrow[NO], lcol[NO];
+  unsigned kgo[NO], vgo[NO];
+#pragma unroll
+  for (int u = 0; u < NO; ++u) {
+    const int c = tid + u * NT;
+    lrow[u] = c / CPR;
+    lcol[u] = (c - lrow[u] * CPR) * 8;
+    if (!kStep && CH % NT != 0) lrow[u] = min(lrow[u], 63);
+    const int col = min(lcol[u], d - 8);
+    kgo[u] = lrow[u] * (unsigned)p.sk[1] + col;
+    vgo[u] = lrow[u] * (unsigned)p.sv[1] + col;
+  }
+  auto row_of = [&](int u) { return kStep ? lrow[0] + u * RS : lrow[kStep ? 0 : u]; };
+  auto in = [&](int u) { return (kStep || CH % NT == 0 || tid + u * NT < CH) && lcol[kStep ? 0 : u] < d; };
+  auto partial = [&](int t) { return (t << 6) + 64 > kend; };
+  auto load_tile = [&](const T* base, const long* st, const unsigned* off, int t, u32x4* reg) {
+    if (!partial(t) && !wide) {
+      const T* tb = base + (long)(t << 6) * st[1];
+#pragma unroll
+      for (int u = 0; u < PT; ++u)
+        reg[u] = *reinterpret_cast<const u32x4*>(tb + (kStep ? u * RS * st[1] : 0) + off[kStep ? 0 : u]);
+    } else {
+#pragma unroll
+      for (int u = 0; u < PT; ++u) {
+        const int row = min((t << 6) + row_of(u), kend - 1);
+        reg[u] = *reinterpret_cast<const u32x4*>(base + (long)row * st[1] + min(lcol[kStep ? 0 : u], d - 8));
+      }
+    }
+  };
   u32x4 kreg[PT], vreg[PT];
-  bool kok[PT], vok[PT];
-  auto load_k = [&](int t) {
+  auto load_k = [&](int t) { load_tile(kbase, p.sk, kgo, t, kreg); };
+  auto load_v = [&](int t) { load_tile(vbase, p.sv, vgo, t, vreg); };
+  auto store_tile = [&](T* buf, int stride, const u32x4* reg) {
 #pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int c = tid + u * NT;
-      const int r = c / CPR, c8 = (c % CPR) * 8;
-      const int key = (t << 6) + r;
-      const bool ok = (CH % NT == 0 || c < CH) && key < kend && c8 < d;
-      kok[u] = ok;
-      kreg[u] = *reinterpret_cast<const u32x4*>(kbase + (ok ? (long)key * p.sk[1] + c8 : 0));
-    }
+    for (int u = 0; u < PT; ++u)
+      if (in(u)) *reinterpret_cast<u32x4*>(buf + row_of(u) * stride + lcol[kStep ? 0 : u]) = reg[u];
   };
-  auto load_v = [&](int t) {
+  auto store_k = [&](int buf) { store_tile(ks_base + buf * KBUF, KSTR, kreg); };
+  auto store_v = [&](int t, int buf) {
+    if (partial(t)) {
 #pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int c = tid + u * NT;
-      const int r = c / CPR, c8 = (c % CPR) * 8;
-      const int key = (t << 6) + r;
-      const bool ok = (CH % NT == 0 || c < CH) && key < kend && c8 < d;
-      vok[u] = ok;
-      vreg[u] = *reinterpret_cast<const u32x4*>(vbase + (ok ? (long)key * p.sv[1] + c8 : 0));
+      for (int u = 0; u < PT; ++u)
+        if ((t << 6) + row_of(u) >= kend) vreg[u] = u32x4{};
     }
+    store_tile(vs_base + buf * VBUF, VSTR, vreg);
   };
-  auto store_k = [&](int buf) {
-    T* kb = ks_base + buf * KBUF;
-#pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int c = tid + u * NT;
-      if (CH % NT == 0 || c < CH)
-        *reinterpret_cast<u32x4*>(kb + (c / CPR) * KSTR + (c % CPR) * 8) = kok[u] ? kreg[u] : u32x4{};
+  if (d < DP) {  // K columns past d multiply zeros of q, so they must be finite; V's only feed rows that are dropped
+    for (int c = tid; c < 2 * CH; c += NT) {
+      const int r = c / CPR, c8 = c % CPR * 8;
+      if (c8 >= d) *reinterpret_cast<u32x4*>(ks_base + (r >> 6) * KBUF + (r & 63) * KSTR + c8) = u32x4{};
     }
-  };
-  auto store_v = [&](int buf) {
-    T* vb = vs_base + buf * VBUF;
-#pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int c = tid + u * NT;
-      if (CH % NT == 0 || c < CH)
-        *reinterpret_cast<u32x4*>(vb + (c / CPR) * VSTR + (c % CPR) * 8) = vok[u] ? vreg[u] : u32x4{};
-    }
-  };
+  }
 
   // The first K and V tiles, the second K tile (in a register set of its own) and the Q fragments are
   // all in flight together, so that the key loop starts one memory latency after the workgroup does
@@ -162,19 +195,7 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
   load_k(t_begin);
   load_v(t_begin);
   u32x4 kreg1[PT];
-  bool kok1[PT];
-  {
-    const int t1 = min(t_begin + 1, tl);
-#pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int c = tid + u * NT;
-      const int r = c / CPR, c8 = (c % CPR) * 8;
-      const int key = (t1 << 6) + r;
-      const bool ok = (CH % NT == 0 || c < CH) && key < kend && c8 < d;
-      kok1[u] = ok;
-      kreg1[u] = *reinterpret_cast<const u32x4*>(kbase + (ok ? (long)key * p.sk[1] + c8 : 0));
-    }
-  }
+  load_tile(kbase, p.sk, kgo, min(t_begin + 1, tl), kreg1);
 
   // Q fragments (B operand of S^T = K Q^T): lane supplies Q[query n][16*s + 8*hh + j], j = 0..7
   X8 qf[KS];
@@ -202,16 +223,8 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
     qf[s] = val;
   }
   store_k(0);
-  store_v(0);
-  {
-    T* kb = ks_base + KBUF;
-#pragma unroll
-    for (int u = 0; u < PT; ++u) {
-      const int c = tid + u * NT;
-      if (CH % NT == 0 || c < CH)
-        *reinterpret_cast<u32x4*>(kb + (c / CPR) * KSTR + (c % CPR) * 8) = kok1[u] ? kreg1[u] : u32x4{};
-    }
-  }
+  store_v(t_begin, 0);
+  store_tile(ks_base + KBUF, KSTR, kreg1);
   __syncthreads();
 
   // per-lane constant parts of the LDS addresses
@@ -247,15 +260,43 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
     }
   };
 
+  // The mask of tile t at this lane's query and keys, four keys at a time where they are adjacent (any
+  // alignment); 0 past the last key.
+  auto load_mask = [&](int t, float (*mv)[16]) {
+    typedef typename Vec<T>::x4 __attribute__((aligned(2))) X4U;
+    const T* mrow = reinterpret_cast<const T*>(p.mask) + bi * p.sm[0] + head * p.sm[1] +
+                    (long)(qvalid ? qidx : 0) * p.sm[2];
+#pragma unroll
+    for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const int k0 = (t << 6) + 32 * mb + 8 * a;  // keys k0 .. k0 + 7, four to a lane half
+        if (p.sm[3] == 1 && k0 + 8 <= kend) {
+          const typename Vec<T>::x4 x = *reinterpret_cast<const X4U*>(mrow + k0 + 4 * hh);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) mv[mb][4 * a + j] = to_f32(x[j]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const int key = k0 + 4 * hh + j;
+            mv[mb][4 * a + j] = key < kend ? to_f32(mrow[(long)key * p.sm[3]]) : 0.f;
+          }
+        }
+      }
+  };
+
   // Softmax and P.V of tile t (scores in s_cur, buffers t&1) with the S^T of tile t+1 into s_nxt.
   // Past the last tile the loads and the next S^T run on clamped indices and their results go unused.
   auto step = [&](int t, f32x16* s_cur, f32x16* s_nxt) {
     const int i = t - t_begin;
     load_k(min(t + 2, tl));
-    X8 b[4], blo[4];
-    {
+    if (!kLateV) load_v(min(t + 1, tl));
+    if (active) {
+      X8 b[4], blo[4];
+      float mv[2][16];
+      if constexpr (MASK) load_mask(t, mv);
       // keys past the end of the last tile: -inf scores
-      if ((t << 6) + 64 > kend) {
+      if (partial(t)) {
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
@@ -265,16 +306,10 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
       if constexpr (MASK) {
         // sdpa's additive mask (sam3/nn.rs:29-32) joins the scaled scores in log2 units:
         // s <- s * scale * log2(e) + mask * log2(e); the softmax below then takes s as it is
-        const T* mrow = reinterpret_cast<const T*>(p.mask) + bi * p.sm[0] + head * p.sm[1] +
-                        (long)(qvalid ? qidx : 0) * p.sm[2];
 #pragma unroll
         for (int mb = 0; mb < 2; ++mb)
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            const int key = (t << 6) + 32 * mb + 8 * (e >> 2) + 4 * hh + (e & 3);
-            const float mv = key < kend ? to_f32(mrow[(long)key * p.sm[3]]) : 0.f;
-            s_cur[mb][e] = fmaf(s_cur[mb][e], sc, mv * kFlashLog2e);
-          }
+          for (int e = 0; e < 16; ++e) s_cur[mb][e] = fmaf(s_cur[mb][e], sc, mv[mb][e] * kFlashLog2e);
       }
       float mm = s_cur[0][0];
 #pragma unroll
@@ -304,15 +339,12 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
         float pv[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) pv[j] = exp2_fast(fmaf(s_cur[u >> 1][8 * (u & 1) + j], scs, c));
-        b[u] = pack8(pv, (X8*)nullptr);
         if constexpr (kSplitP) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            lsum += pv[j];
-            pv[j] -= to_f32(b[u][j]);
-          }
-          blo[u] = pack8(pv, (X8*)nullptr);
+          for (int j = 0; j < 8; ++j) lsum += pv[j];
+          split_hi_lo(pv, b[u], blo[u]);
         } else {
+          b[u] = pack8(pv, (X8*)nullptr);
           typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 #pragma unroll
           for (int j = 0; j < 8; j += 2)
@@ -320,12 +352,6 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
         }
       }
       l_run += lsum;
-    }
-    // K(t+2) replaces K(t), whose scores were taken one step ago; only then is V(t+1) fetched, so at
-    // most one tile's staging registers are live
-    store_k(i & 1);
-    load_v(min(t + 1, tl));
-    {
       // O^T += V^T . P^T; in bf16, P is split into hi + lo bf16 terms so the product keeps ~16 bits of P
       const T* vb = vs_base + (i & 1) * VBUF;
 #pragma unroll
@@ -340,20 +366,20 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
         }
       }
     }
-    store_v((i + 1) & 1);  // V(t+1) replaces V(t-1)
+    if (kLateV) load_v(min(t + 1, tl));
+    // K(t+2) replaces K(t), whose scores were taken one step ago, V(t+1) replaces V(t-1)
+    store_k(i & 1);
+    store_v(min(t + 1, tl), (i + 1) & 1);
     __syncthreads();
   };
 
-  // A wave whose 32 queries are all past the end computes on zero queries (no divergent branch in the
-  // loop) and stores nothing.
   f32x16 sa[2], sb[2];
-  qk(ks_base, sa);
+  if (active) qk(ks_base, sa);  // a wave whose 32 queries are all past the end only stages
   __syncthreads();  // every wave has read K(0) before step 0 overwrites its buffer with K(2)
   for (int t = t_begin; t < t_end; t += 2) {
     step(t, sa, sb);
     if (t + 1 < t_end) step(t + 1, sb, sa);
   }
-  (void)ntiles;
 
   if (!active) return;
   // lane holds O^T[32*ob + 8*a + 4*hh + b][query n]
@@ -375,9 +401,9 @@ __global__ __launch_bounds__(NW * 64, NW == 4 && DP <= 64 && __is_same(T, f16) ?
         }
       }
   } else {
-    // partial O [split][bh][q][DP] (unnormalised, f32) and (max, sum) [split][bh][q][2]
+    // partial O [split][bh][q][PD] (unnormalised, f32) and (max, sum) [split][bh][q][2]
     const long row = ((long)split * p.b * p.h + bhi) * p.lq + qidx;
-    float* prow = p.opart + row * DP;
+    float* prow = p.opart + row * FG::PD;
 #pragma unroll
     for (int ob = 0; ob < MBO; ++ob)
 #pragma unroll
@@ -489,8 +515,8 @@ static hipError_t launch_flash(FlashParams p, bool ropeq, hipStream_t stream) {
   }
   if (e != hipSuccess || p.nsplit == 1) return e;
   const long rows = (long)p.b * p.h * p.lq;
-  constexpr int kRowsPerBlock = 256 / (DP / 8);
-  hipLaunchKernelGGL((flash_combine_kernel<T, DP>), dim3((unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock)),
+  constexpr int kRowsPerBlock = 256 / (FG::PD / 8);
+  hipLaunchKernelGGL((flash_combine_kernel<T, FG::PD>), dim3((unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock)),
                      dim3(256), 0, stream, p);
   return hipGetLastError();
 }
@@ -512,27 +538,38 @@ int flash_queries_per_block(int dtype, int d, int lk) {
 }
 
 // Key splits, at least 2 key tiles per split. 4-wave f16 / bf16 workgroups (three resident per CU in
-// f16 up to head dim 64, two otherwise): as many splits as still fit one round of resident workgroups,
-// none once the query blocks alone fill it. Measured on f16 against other split counts: a short key
-// range (SAM 3's 576-token windows) loses 35% when split in two, and 4096 x 4096 over 16 heads 9%,
-// while 12 heads (384 query blocks) gain 13% from two splits. Otherwise (8 waves, f32, head dim 256):
-// enough workgroups to give every CU its resident share (one workgroup per CU at head dim 256, two
-// below).
+// f16 up to head dim 64, two otherwise): the count that gives the least time among those that fit one round
+// of resident workgroups. A tile takes about 0.85 us (1.1 in bf16) alone on its CU and 0.6 times as much
+// again for each workgroup beside it; merging costs about 3.3 us and 0.5 us per MB of partials. Measured
+// against as many splits as fit, in f16: 64 windows of 256 keys at head dim 72 18.2 -> 9.5 us (1 for 2), 4096 x 4096
+// over one head at 64 26.5 -> 18.5 (8 for 22), 8 heads of 1024 at 64 20.4 -> 14.9 (4 for 8); 12 heads of
+// 4096 keep 2, 13% faster than none, and one of 1024 at 72 its 8 (12.0 us, 16.2 with 2). Otherwise (8 waves,
+// f32, head dim 256): enough workgroups to give every CU its resident share (one workgroup per CU at head
+// dim 256, two below).
 void flash_plan(int dtype, int b, int h, int lq, int lk, int d, int cus, int* qblocks, int* nsplit, int* tps) {
   const int qpb = flash_queries_per_block(dtype, d, lk);
   *qblocks = (lq + qpb - 1) / qpb;
   const int tiles = (lk + 63) / 64;
   const long base = (long)b * h * *qblocks;
   const int dp = flash_padded_dim(d);
+  const int maxs = tiles / 2 > 1 ? tiles / 2 : 1;
   int ns = 1;
   if (dtype != kF32 && dp <= 128 && qpb == 128) {
     const long slots = (long)cus * (dtype == kF16 && dp <= 64 ? 3 : 2);
-    if (base < slots) ns = (int)(slots / base);
+    const float tile = dtype == kF16 ? 0.85f : 1.1f, mb = (float)b * h * lq * dp * 4e-6f;
+    float best = INFINITY;
+    for (int n = 1; n <= maxs && n <= 64 && (n == 1 || n * base <= slots); ++n) {
+      const long beside = (n * base + cus - 1) / cus - 1;
+      const float time = tile * (1.f + 0.6f * beside) * ((tiles + n - 1) / n) + (n > 1 ? 3.3f + 0.5f * mb * n : 0.f);
+      if (time < best) {
+        best = time;
+        ns = n;
+      }
+    }
   } else {
     const long target = (long)cus * (dp <= 128 ? 2 : 1);
     if (base < target) ns = (int)((target + base - 1) / base);
   }
-  const int maxs = tiles / 2 > 1 ? tiles / 2 : 1;
   if (ns > maxs) ns = maxs;
   if (ns > 64) ns = 64;
   int t = (tiles + ns - 1) / ns;
@@ -549,6 +586,8 @@ size_t flash_partial_bytes(int b, int h, int lq, int d, int nsplit) {
 template <typename T>
 static hipError_t flash_dispatch(FlashParams p, bool ropeq, hipStream_t s) {
   const bool four = flash_queries_per_block(__is_same(T, f16) ? kF16 : kBF16, p.d, p.lk) == 128;
+  // 65..80 takes 5 k-steps of 16 instead of 6 (its O rows and partials are those of 96)
+  if (p.d > 64 && p.d <= 80) return four ? launch_flash<T, 80, 4>(p, ropeq, s) : launch_flash<T, 80, 8>(p, ropeq, s);
   switch (flash_padded_dim(p.d)) {
     case 32: return launch_flash<T, 32, 4>(p, ropeq, s);
     case 64: return launch_flash<T, 64, 4>(p, ropeq, s);

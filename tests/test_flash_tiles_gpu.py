@@ -1,0 +1,73 @@
+"""The f16 / bf16 flash kernel's staging, tail and mask paths against attention in 64 bits, on an MI355X: head
+dims around its padded ones, key counts around the tile of 64, row strides whose offsets need 64 bits, and
+masks whose rows start at any element or whose keys are not adjacent."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DT = {"f16": torch.float16, "bf16": torch.bfloat16}
+# P as f16 (2^-11) or as two bf16 terms, and the output's own rounding, over values of deviation 1
+TOL = {"f16": 2e-3, "bf16": 1.2e-2}
+
+
+@pytest.fixture(scope="module")
+def hip():
+    import sam_hip
+
+    sam_hip.load()
+    assert torch.cuda.is_available(), "no GPU visible"
+    return sam_hip
+
+
+def rn(seed, dtype, *shape):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(*shape, device="cuda", generator=g).to(DT[dtype])
+
+
+def exact(q, k, v, mask=None):
+    """softmax(q k^T d^-1/2 + mask) v of [B, H, L, D] in 64 bits."""
+    s = torch.matmul(q.double(), k.double().transpose(2, 3).contiguous()) * q.shape[3] ** -0.5
+    if mask is not None:
+        s = s + mask.double()
+    return torch.matmul(torch.softmax(s, 3), v.double().contiguous())
+
+
+def close(got, want, dtype):
+    err = (got.double() - want).abs().max().item()
+    assert err <= TOL[dtype], err
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("d", [8, 32, 40, 64, 72, 80, 88, 96, 104, 128])
+@pytest.mark.parametrize("lq,lk", [(1, 1), (33, 63), (128, 64), (129, 65), (5, 190), (40, 1090)])
+def test_head_dims_and_tails(hip, d, lq, lk, dtype):
+    print(f"flash tiles {dtype} d={d} {lq}x{lk}", flush=True)
+    q, k, v = (rn(i, dtype, 2, n, 3, d) for i, n in ((1, lq), (2, lk), (3, lk)))
+    want = exact(*(x.transpose(1, 2) for x in (q, k, v))).transpose(1, 2)
+    close(hip.flash_attn(q, k, v), want, dtype)
+
+
+@pytest.mark.parametrize("d", [64, 72])
+def test_row_strides_past_32_bits(hip, d):
+    """A row stride of 2^24 elements and more: the offsets of a tile no longer fit in 32 bits."""
+    n, stride = 3, (1 << 24) + 8
+    q = rn(1, "f16", 1, 20, 1, d)
+    k, v = (torch.empty_strided((1, n, 1, d), (0, stride, d, 1), device="cuda", dtype=torch.float16) for _ in "kv")
+    k.copy_(rn(2, "f16", 1, n, 1, d))
+    v.copy_(rn(3, "f16", 1, n, 1, d))
+    want = exact(*(x.transpose(1, 2) for x in (q, k, v))).transpose(1, 2)
+    close(hip.flash_attn(q, k, v), want, "f16")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("d,lk", [(32, 7), (32, 64), (32, 197), (64, 130), (72, 197)])
+@pytest.mark.parametrize("form", ["rows", "keys", "offset", "transposed"])
+def test_masks(hip, form, d, lk, dtype):
+    """A mask of odd rows, one of keys alone, one that starts at an odd element, and one whose keys are strided."""
+    b, h, lq = 2, 3, 37
+    print(f"flash mask {form} {dtype} d={d} lk={lk}", flush=True)
+    q, k, v = (rn(i, dtype, b, h, n, d) for i, n in ((1, lq), (2, lk), (3, lk)))
+    mask = {"rows": lambda: rn(4, dtype, b, h, lq, lk), "keys": lambda: rn(4, dtype, b, 1, 1, lk),
+            "offset": lambda: rn(4, dtype, h * lq * lk + 1)[1:].view(1, h, lq, lk),
+            "transposed": lambda: rn(4, dtype, b, h, lk, lq).transpose(2, 3)}[form]()
+    close(hip.sdpa(q, k, v, mask), exact(q, k, v, mask), dtype)
