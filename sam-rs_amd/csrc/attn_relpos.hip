@@ -391,7 +391,10 @@ __global__ __launch_bounds__(NWV * 64) void attn_relpos_kernel(const T* __restri
           pv[j] = exp2_fast(POS ? fmaf(x, sc, c[u >> 1]) : x + c[u >> 1]);
           if (!kOnes && kSplitP) lsum += pv[j];  // bf16: P.V takes hi + lo, P itself to ~16 bits
         }
-        b[u] = pack8(pv, (X8*)nullptr);
+        if constexpr (kSplitP)
+          split_hi_lo(pv, b[u], blo[u]);
+        else
+          b[u] = pack8(pv, (X8*)nullptr);
         if constexpr (!kOnes && !kSplitP) {
           // f16: the sum over P as the P.V product sees it (rounded), as the ones row gives it when hd
           // leaves a spare O^T row: numerator and denominator weigh each key alike
@@ -399,11 +402,6 @@ __global__ __launch_bounds__(NWV * 64) void attn_relpos_kernel(const T* __restri
 #pragma unroll
           for (int j = 0; j < 8; j += 2)
             lsum = __builtin_amdgcn_fdot2(h2{b[u][j], b[u][j + 1]}, h2{(f16)1.f, (f16)1.f}, lsum, false);
-        }
-        if (kSplitP) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) pv[j] -= to_f32(b[u][j]);
-          blo[u] = pack8(pv, (X8*)nullptr);
         }
       }
       if (!kOnes) l_run += lsum;

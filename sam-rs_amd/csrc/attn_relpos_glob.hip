@@ -322,7 +322,10 @@ __global__ __launch_bounds__(glob::kThreads) void attn_relpos_glob_kernel(const 
         const float x = s_cur[w4 >> 1][8 * (w4 & 1) + e];
         pv[e] = exp2_fast(fmaf(x, sc, cc));
       }
-      b[w4] = pack8(pv, (X8*)nullptr);
+      if constexpr (kSplitP)
+        split_hi_lo(pv, b[w4], blo[w4]);
+      else
+        b[w4] = pack8(pv, (X8*)nullptr);
       if constexpr (!S::kOnesRows) {
         if constexpr (kF16) {
           typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -333,11 +336,6 @@ __global__ __launch_bounds__(glob::kThreads) void attn_relpos_glob_kernel(const 
 #pragma unroll
           for (int e = 0; e < 8; ++e) lsum += pv[e];
         }
-      }
-      if (kSplitP) {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) pv[e] -= to_f32(b[w4][e]);
-        blo[w4] = pack8(pv, (X8*)nullptr);
       }
     }
 #pragma unroll

@@ -323,7 +323,10 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
         float pv[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) pv[e] = exp2_fast(fmaf(s_cur[w4 >> 1][8 * (w4 & 1) + e], sc, -m_run));
-        b[w4] = pack8(pv, (X8*)nullptr);
+        if constexpr (kSplitP)
+          split_hi_lo(pv, b[w4], blo[w4]);
+        else
+          b[w4] = pack8(pv, (X8*)nullptr);
         if constexpr (!S::kOnesRow) {
           if constexpr (!kSplitP) {
             // f16: the sum over P as the P.V product sees it (rounded)
@@ -335,11 +338,6 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
 #pragma unroll
             for (int e = 0; e < 8; ++e) l_run += pv[e];
           }
-        }
-        if (kSplitP) {
-#pragma unroll
-          for (int e = 0; e < 8; ++e) pv[e] -= to_f32(b[w4][e]);
-          blo[w4] = pack8(pv, (X8*)nullptr);
         }
       }
       const T* vp = vl + (t & 1) * S::kVBuf;

@@ -312,7 +312,10 @@ __global__ __launch_bounds__(NW * 64) void attn_relpos_wide_kernel(const T* __re
           pv[j] = exp2_fast(POS ? fmaf(x, sc, c) : x + c);
           if (!kOnes && kSplitP) lsum += pv[j];  // bf16: P.V takes hi + lo, P itself to ~16 bits
         }
-        b[u] = pack8(pv, (X8*)nullptr);
+        if constexpr (kSplitP)
+          split_hi_lo(pv, b[u], blo[u]);
+        else
+          b[u] = pack8(pv, (X8*)nullptr);
         if constexpr (!kOnes && !kSplitP) {
           // f16: the sum over P as the P.V product sees it (rounded), so that numerator and
           // denominator weigh each key alike (the ones row does the same when hd leaves one spare):
@@ -321,11 +324,6 @@ __global__ __launch_bounds__(NW * 64) void attn_relpos_wide_kernel(const T* __re
 #pragma unroll
           for (int j = 0; j < 8; j += 2)
             lsum = __builtin_amdgcn_fdot2(h2{b[u][j], b[u][j + 1]}, h2{(f16)1.f, (f16)1.f}, lsum, false);
-        }
-        if (kSplitP) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) pv[j] -= to_f32(b[u][j]);
-          blo[u] = pack8(pv, (X8*)nullptr);
         }
       }
       if (!kOnes) l_run += lsum;

@@ -237,15 +237,12 @@ __global__ __launch_bounds__(f256::kThreads) void flash256_kernel(FlashParams p)
         float pv[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) pv[j] = exp2_fast(fmaf(s[2 * u + (j >> 2)][j & 3], p.sc, c));
-        b[u] = pack8(pv, (X8*)nullptr);
         if constexpr (kSplitP) {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            lsum += pv[j];
-            pv[j] -= to_f32(b[u][j]);
-          }
-          blo[u] = pack8(pv, (X8*)nullptr);
+          for (int j = 0; j < 8; ++j) lsum += pv[j];
+          split_hi_lo(pv, b[u], blo[u]);
         } else {
+          b[u] = pack8(pv, (X8*)nullptr);
           typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 #pragma unroll
           for (int j = 0; j < 8; j += 2)
