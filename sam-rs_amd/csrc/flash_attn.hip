@@ -69,11 +69,9 @@ __device__ __forceinline__ void rope_pair(float x0, float x1, float c0, float s0
   y1 = x1 * c1 + x0 * s1;
 }
 
-template <typename T, int DP, int NW, bool MASK>
-constexpr bool kThreePerSimd = NW == 4 && DP <= 64 && __is_same(T, f16) && !(DP == 64 && MASK);
-
-// f16 4-wave workgroups (head dims up to 64) are held to 168 registers, so that three share a CU (bf16,
-// whose P.V takes P as hi + lo, would spill there and runs two to a CU). Up to head dim 128 the others are
+// THREE: held to 168 registers, so that three 4-wave workgroups share a CU (f16 up to head dim 64; bf16, whose
+// P.V takes P as hi + lo, would spill). At head dim 64 that leaves no room to fetch V a tile ahead, so a launch
+// of at most two workgroups per CU takes the instance without. Up to head dim 128 the others are
 // held to 256 in all: without that bound the compiler keeps O in accumulation registers and copies it out
 // and back around the rescale.
 //
@@ -84,14 +82,14 @@ constexpr bool kThreePerSimd = NW == 4 && DP <= 64 && __is_same(T, f16) && !(DP 
 // packed conversions; a wave without queries only stages. 64 x 4 windows of 196 at head dim 72, bf16: 23.4 us
 // at 2613 VALU instructions a wave before, now 17.2 (f16 21.4 -> 14.6); 128 heads of 1024 at 96, f16 106.6 ->
 // 74.5; 144 of 576 at 64 28.9 -> 27.3 (bf16 36.2 -> 31.9); with a 196 x 196 bias, 320 heads at 32 31.1 -> 17.5.
-template <typename T, int DP, int NW, bool ROPEQ, bool MASK>
-__global__ __launch_bounds__(NW * 64, (kThreePerSimd<T, DP, NW, MASK> ? 3 : DP <= 128 ? 2 : 1)) void flash_fwd_kernel(
+template <typename T, int DP, int NW, bool ROPEQ, bool MASK, bool THREE>
+__global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flash_fwd_kernel(
     FlashParams p) {
   typedef FlashGeom<T, DP, NW> FG;
   typedef typename Vec<T>::x8 X8;
   constexpr bool kSplitP = __is_same(T, bf16);
   // at 168 registers there is no room for V(t+1) beside the scores; the other two waves cover its latency
-  constexpr bool kLateV = kThreePerSimd<T, DP, NW, MASK> && DP == 64;
+  constexpr bool kLateV = THREE && DP == 64;
   constexpr int KS = FG::KS, MBO = FG::MBO, KSTR = FG::KSTR, VSTR = FG::VSTR;
   constexpr int KBUF = FG::KBUF, VBUF = FG::VBUF, NT = FG::NT;
   constexpr int CPR = FG::CPR, CH = FG::CH, PT = FG::PT;
@@ -502,14 +500,22 @@ static hipError_t launch_flash(FlashParams p, bool ropeq, hipStream_t stream) {
   if (DP == 256 && !p.mask && flash256_eligible(p, (int)sizeof(T))) {
     e = flash256_launch(__is_same(T, f16) ? kF16 : kBF16, p, ropeq, stream);
   } else {
-    const int which = p.mask ? 2 : ropeq ? 1 : 0;  // a masked call has no RoPE
-    auto kern = which == 2   ? flash_fwd_kernel<T, DP, NW, false, true>
-                : which == 1 ? flash_fwd_kernel<T, DP, NW, true, false>
-                             : flash_fwd_kernel<T, DP, NW, false, false>;
-    static std::atomic<unsigned long long> lds_done[3];  // opt-in to more than 64 KB of dynamic LDS
+    // Three workgroups per CU with V fetched late, or two with V a tile ahead, f16 at head dim 64 (one SAM 3
+    // layer): 256 workgroups of 32 tiles 56 / 44 us, 416 of 25 52 / 49, 512 of 64 109 / 103, 656 of 81 163 / 187,
+    // 720 of 9 39 / 42.
+    constexpr bool kHalf3 = NW == 4 && DP <= 64 && __is_same(T, f16);
+    const long blocks = (long)p.b * p.h * p.qblocks * p.nsplit;
+    const bool three = kHalf3 && (DP < 64 || (!p.mask && blocks > 2L * device_cu_count()));
+    const int which = (p.mask ? 2 : ropeq ? 1 : 0) + (three && DP == 64 ? 3 : 0);  // a masked call has no RoPE
+    constexpr bool k3 = kHalf3 && DP < 64;  // the only form there is
+    auto kern = which == 0   ? flash_fwd_kernel<T, DP, NW, false, false, k3>
+                : which == 1 ? flash_fwd_kernel<T, DP, NW, true, false, k3>
+                : which == 2 ? flash_fwd_kernel<T, DP, NW, false, true, k3>
+                : which == 3 ? flash_fwd_kernel<T, DP, NW, false, false, kHalf3>
+                             : flash_fwd_kernel<T, DP, NW, true, false, kHalf3>;
+    static std::atomic<unsigned long long> lds_done[5];  // opt-in to more than 64 KB of dynamic LDS
     e = lds_opt_in(lds_done[which], (const void*)kern, (int)FG::LDS);
     if (e != hipSuccess) return e;
-    const long blocks = (long)p.b * p.h * p.qblocks * p.nsplit;
     hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(FG::NT), FG::LDS, stream, p);
     e = hipGetLastError();
   }
