@@ -156,6 +156,27 @@ __global__ __launch_bounds__(ff32::Geom<DP>::NT) void flash_f32_kernel(FlashPara
     const bool more = k0 + 32 < k_end;
     if (more) load_tile(k0 + 32);  // in flight while tile k0 is computed
     if (active) {
+      // the mask, ahead of the products that hide its latency: four keys at a time where they are adjacent
+      // (one by one after the products: 320 heads of 196 x 196 at head dim 32 took 68.8 us, now 52.0)
+      float mv[16];
+      if constexpr (MASK) {
+        typedef f32x4 __attribute__((aligned(4))) f32x4_a4;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          const int ka = k0 + 8 * a;  // keys ka .. ka + 7, four to a lane half
+          if (p.sm[3] == 1 && ka + 8 <= kend) {
+            const f32x4 x = *reinterpret_cast<const f32x4_a4*>(mrow + ka + 4 * hh);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) mv[4 * a + e] = x[e];
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+              const int key = ka + 4 * hh + e;
+              mv[4 * a + e] = key < kend ? mrow[(long)key * p.sm[3]] : 0.f;
+            }
+          }
+        }
+      }
       // S^T: lane holds key k0 + 8 (i / 4) + 4 hh + (i % 4) for query n in s[i]
       f32x16 s = f32x16{};
       const float* krow = ks + n * KSTR + HALF * hh;
@@ -171,7 +192,7 @@ __global__ __launch_bounds__(ff32::Geom<DP>::NT) void flash_f32_kernel(FlashPara
       for (int i = 0; i < 16; ++i) {
         const int key = k0 + 8 * (i >> 2) + 4 * hh + (i & 3);
         float x = s[i] * scale;
-        if constexpr (MASK) x = key < kend ? x + mrow[(long)key * p.sm[3]] : x;
+        if constexpr (MASK) x = x + mv[i];
         s[i] = key < kend ? x : -INFINITY;
         mm = fmaxf(mm, s[i]);
       }

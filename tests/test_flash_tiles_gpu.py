@@ -1,13 +1,13 @@
-"""The f16 / bf16 flash kernel's staging, tail and mask paths against attention in 64 bits, on an MI355X: head
+"""The flash kernels' staging, tail and (f32 too) mask paths against attention in 64 bits, on an MI355X: head
 dims around its padded ones, key counts around the tile of 64, row strides whose offsets need 64 bits, and
 masks whose rows start at any element or whose keys are not adjacent."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
-DT = {"f16": torch.float16, "bf16": torch.bfloat16}
-# P as f16 (2^-11) or as two bf16 terms, and the output's own rounding, over values of deviation 1
-TOL = {"f16": 2e-3, "bf16": 1.2e-2}
+DT = {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}
+# P as f16 (2^-11) or as two bf16 terms, and the output's own rounding, over values of deviation 1; f32: the sums'
+TOL = {"f16": 2e-3, "bf16": 1.2e-2, "f32": 1e-5}
 
 
 @pytest.fixture(scope="module")
@@ -59,7 +59,7 @@ def test_row_strides_past_32_bits(hip, d):
     close(hip.flash_attn(q, k, v), want, "f16")
 
 
-@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
 @pytest.mark.parametrize("d,lk", [(32, 7), (32, 64), (32, 197), (64, 130), (72, 197)])
 @pytest.mark.parametrize("form", ["rows", "keys", "offset", "transposed"])
 def test_masks(hip, form, d, lk, dtype):
