@@ -25,6 +25,7 @@
 
 #include "lds_dma.hpp"
 #include "relpos_geom.hpp"
+#include "rows_tiles.hpp"
 
 namespace samhip {
 
@@ -42,9 +43,6 @@ template <int HD> struct Shape {
   static constexpr int kVBuf = 64 * kVStride;
   static constexpr int kTiles = 2 * (kKBuf + kVBuf);  // elements per wave group: two K and two V buffers
 };
-
-constexpr int gcd8(int c) { return c % 8 == 0 ? 8 : (c % 4 == 0 ? 4 : (c % 2 == 0 ? 2 : 1)); }
-constexpr int period(int cpr) { return cpr / gcd8(cpr); }  // tiles after which the chunk pattern repeats
 
 __device__ __forceinline__ int xcd_block(int i, int total) {
   const int per = total >> 3, rem = total & 7, x = i & 7, j = i >> 3;
@@ -100,8 +98,8 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
   // 8 t = (row 8 t / CPR, column group phase); a thread's chunk is a fixed distance from there, so its
   // offset is a few operations on constants of the phase, and the rest is a wave-uniform base.
   //   K: chunk gt % 8 of hd rows gt / 8 + u * kGT / 8. The columns of a row's last chunk past W are the next
-  //   grid row's: real keys of this head, masked by the bias. Only where there is no next row (tiles that
-  //   hold the last one) are they cleared, and a load past the head's end starts earlier and is shifted.
+  //   grid row's: real keys of this head, masked by the bias. Only in tiles with chunks that can reach past
+  //   the head's end (first_end_row) are they cleared, and a load past that end starts earlier and is shifted.
   //   V: slot gt / kTPS, 16-byte pieces gt % kTPS + u * kTPS. Columns past W and rows past the group's are
   //   out of the buffer's range, which reads 0.
   constexpr int KPT = (HD * 8 + kGT - 1) / kGT;
@@ -117,19 +115,12 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
   const bool vtail = (vsl & 7) < tailcols;
   const auto vrsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<T*>(v + (bh * N + r0 * W) * (long)HD), 0, (int)((r1 - r0) * W * HD * sizeof(T)), 0x00020000);
-  // whether tile t reaches the last grid row (either group's: the first reads on past its rows)
-  auto has_end = [&](int t) { return 8 * t + 8 > (H - 1 - r0) * CPR; };
-  // elements by which the K load of hd row d at column offset x starts early
-  auto k_early = [&](int d, int x) {
-    const int over = d * N + x + 8 - HD * N;
-    return over > 0 ? over : 0;
-  };
+  // whether a K load of tile t can pass the head's end (either group's: the first reads on past its rows)
+  const int first_end = first_end_row(H, W, CPR);
+  auto has_end = [&](int t) { return reaches_row(t, r0, first_end, CPR); };
   auto k_x = [&](int t, auto uc) {
     constexpr int j0 = (8 * decltype(uc)::value) % CPR;
-    const int j = j0 + (int)opaque(kj);  // opaque: computed here, not held in a register per phase
-    const int add = j / CPR, cc = j - add * CPR;
-    const int row = r0 + (8 * t) / CPR + add;
-    return (row < H ? row : H - 1) * W + 8 * cc;
+    return k_column(t, j0, (int)opaque(kj), r0, H, W, CPR);  // opaque: computed here, not held in a register per phase
   };
   auto load_k = [&](int t, auto uc) {
     const int x = k_x(t, uc);
@@ -138,7 +129,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
     for (int u = 0; u < KPT; ++u) {
       if (u + 1 < KPT || kpart) {
         unsigned off = (unsigned)(kd * N + x);
-        if (end) off -= (unsigned)k_early(kd + u * (kGT / 8), x);
+        if (end) off -= (unsigned)k_early(kd + u * (kGT / 8), x, N, HD);
         const char* base = reinterpret_cast<const char*>(ktb + (long)u * (kGT / 8) * N);
         kreg[u] = *reinterpret_cast<const u32x4_a2*>(base + off * (unsigned)sizeof(T));
       }
@@ -164,7 +155,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
       const bool tail = (j0 + kj) % CPR == CPR - 1;
 #pragma unroll
       for (int u = 0; u < KPT; ++u) {
-        const int early = k_early(kd + u * (kGT / 8), x);
+        const int early = k_early(kd + u * (kGT / 8), x, N, HD);
         if (wave_any(early > 0)) {
           const unsigned long lo = ((unsigned long)kreg[u][1] << 32) | kreg[u][0];
           const unsigned long hi = ((unsigned long)kreg[u][3] << 32) | kreg[u][2];

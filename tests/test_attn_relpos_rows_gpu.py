@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import sam_oracle as oracle
-from parity import check
+from parity import check, to_dev
 from test_attn_relpos_gpu import hip, make_inputs, run_gpu  # noqa: F401
 
 pytestmark = pytest.mark.gpu
@@ -42,4 +42,35 @@ def test_packed_rows_keep_a_head_to_itself(hip, h, w):  # noqa: F811
     kt[1], v[1] = float("nan"), float("nan")
     got = run_gpu(hip, [q, kt, v, table], h, w, hd ** -0.5, "f16")
     assert (got[[0, 2]] == clean[[0, 2]]).all()
+    assert torch.from_numpy(got[1]).isnan().all()
+
+
+# Grids of 1 to 3 columns, where a chunk of 8 spans several rows and the loads of more than the last row's tile
+# reach the head's end: one wave group (up to 128 tokens; 300 heads), and two.
+NARROW = [(9, 1, 3), (12, 1, 3), (10, 2, 3), (9, 3, 3), (17, 3, 3), (49, 3, 3), (51, 3, 3), (51, 3, 300)]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("h,w,bh", NARROW)
+def test_narrow_grids_read_nothing_past_a_head(hip, h, w, bh, hd, dtype):  # noqa: F811
+    """NaN keys and values in one head, and past the last one, must not reach any other head."""
+    print(f"narrow {dtype} {h}x{w} bh={bh} hd={hd}", flush=True)
+    arrays = make_inputs(h, w, bh, hd, 40 + h + w + hd, dtype, table_std=0.5)
+    q, kt, v, table = (to_dev(a, dtype) for a in arrays)
+
+    def tailed(x):
+        buf = torch.full((x.numel() + 4096,), float("nan"), device="cuda", dtype=x.dtype)
+        buf[: x.numel()].copy_(x.reshape(-1))
+        return buf[: x.numel()].view(x.shape)
+
+    kt, v = tailed(kt), tailed(v)
+    clean = hip.attention_relpos(q, kt, v, table, h, w, hd ** -0.5).float().cpu().numpy()
+    heads = [0, bh - 1]
+    want = oracle.attention_relpos(*(a[heads] for a in arrays[:3]), arrays[3], h, w, hd ** -0.5)
+    check(clean[heads], want, dtype, f"narrow {h}x{w} hd={hd} {dtype}")
+    kt[1], v[1] = float("nan"), float("nan")
+    got = hip.attention_relpos(q, kt, v, table, h, w, hd ** -0.5).float().cpu().numpy()
+    rest = [b for b in range(bh) if b != 1]
+    assert (got[rest] == clean[rest]).all()
     assert torch.from_numpy(got[1]).isnan().all()
