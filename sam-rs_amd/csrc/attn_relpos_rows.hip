@@ -141,7 +141,7 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
     const int j = j0 + (sl >> 3), add = j / CPR, cc = j - add * CPR;
     const bool ok = cc < CPR - 1 || vtail;
     const int off = ok ? (int)(((add * W + 8 * cc + (sl & 7)) * HD + 8 * vpc) * sizeof(T)) : 0x40000000;
-    const int base = (int)(((8 * t) / CPR) * W * HD * sizeof(T));
+    const int base = (int)(v_row(t, r1 - r0, CPR) * W * HD * sizeof(T));
 #pragma unroll
     for (int u = 0; u < VPT; ++u)
       if (u + 1 < VPT || vpart)

@@ -32,6 +32,12 @@ constexpr int k_early(int d, int x, int N, int hd) {
   const int over = d * N + x + 8 - hd * N;
   return over > 0 ? over : 0;
 }
+// first V row of tile t in a group of `rows` grid rows: the range check of a buffer load subtracts the uniform
+// offset from the buffer's size, so the tile past the last one (a prefetch) starts at the group's end, no later
+constexpr int v_row(int t, int rows, int cpr) {
+  const int r = 8 * t / cpr;
+  return r < rows ? r : rows;
+}
 
 }  // namespace rows
 }  // namespace samhip

@@ -50,6 +50,51 @@ int main() {
 """
 
 
+V_LOADS = r"""
+#include <cstdio>
+#include "rows_tiles.hpp"
+using namespace samhip::rows;
+
+// The V loads of one wave group of `rows` grid rows, through a descriptor of rows * W * hd elements: the uniform
+// offset must not pass its size (the check is offset >= size - uniform offset, and says nothing of a negative
+// difference); slots past the row's W columns are sent out of range by the caller.
+static int check(int H, int W, int hd, int rows, int ntiles) {
+  const int cpr = (W + 7) / 8, size = rows * W * hd;
+  for (int t = 0; t <= ntiles; ++t) {
+    const int base = v_row(t, rows, cpr) * W * hd;
+    bool ok = base <= size;
+    for (int j = 0; j < 8 && ok; ++j) {
+      const int chunk = 8 * t % cpr + j, add = chunk / cpr, cc = chunk % cpr, row = 8 * t / cpr + add;
+      for (int c = 0; c < 8 && 8 * cc + c < W; ++c) {
+        const int off = (add * W + 8 * cc + c) * hd;
+        // a row of the group is read at its place, any other is out of range
+        ok = ok && (row < rows ? base + off == (row * W + 8 * cc + c) * hd && off < size - base : off >= size - base);
+      }
+    }
+    if (!ok) {
+      printf("H=%d W=%d hd=%d rows=%d tile %d of %d: base %d, size %d\n", H, W, hd, rows, t, ntiles, base, size);
+      return 1;
+    }
+  }
+  return 0;
+}
+
+int main() {
+  int bad = 0;
+  for (int hd = 64; hd <= 80; hd += 16)
+    for (int H = 1; H <= 64; ++H)
+      for (int W = 1; W <= 64; ++W) {
+        const int cpr = (W + 7) / 8, half = (H + 1) / 2;
+        bad += check(H, W, hd, H, (H * cpr + 7) / 8);
+        bad += check(H, W, hd, half, (half * cpr + 7) / 8);
+        if (H > 1) bad += check(H, W, hd, H - half, (half * cpr + 7) / 8);
+      }
+  printf("%d\n", bad);
+  return bad != 0;
+}
+"""
+
+
 def run(tmp_path, source):
     src, exe = tmp_path / "walk.cpp", tmp_path / "walk"
     src.write_text(source)
@@ -61,3 +106,7 @@ def run(tmp_path, source):
 
 def test_k_loads_stay_in_the_head(tmp_path):
     run(tmp_path, K_LOADS)
+
+
+def test_v_loads_stay_in_the_descriptor(tmp_path):
+    run(tmp_path, V_LOADS)
