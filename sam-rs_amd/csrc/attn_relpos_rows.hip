@@ -302,18 +302,20 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
       const float mt = max_with_partner32(mm * sc);
       if (wave_any(mt > m_run + kSlack)) {
         const float m_new = fmaxf(m_run, mt);
-        const float alpha = exp2_fast(m_run - m_new);
+        const float alpha = m_run == -INFINITY ? 0.f : exp2_fast(m_run - m_new);
         l_run *= alpha;
 #pragma unroll
         for (int ob = 0; ob < kMBO; ++ob) o[ob] *= alpha;
         m_run = m_new;
       }
+      // infinite keys: all of a query's scores in a group's tiles so far can be -inf (weight 0)
+      const float c = m_run == -INFINITY ? 0.f : -m_run;
       X8 b[4], blo[4];
 #pragma unroll
       for (int w4 = 0; w4 < 4; ++w4) {
         float pv[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) pv[e] = exp2_fast(fmaf(s_cur[w4 >> 1][8 * (w4 & 1) + e], sc, -m_run));
+        for (int e = 0; e < 8; ++e) pv[e] = exp2_fast(fmaf(s_cur[w4 >> 1][8 * (w4 & 1) + e], sc, c));
         if constexpr (kSplitP)
           split_hi_lo(pv, b[w4], blo[w4]);
         else

@@ -1,5 +1,6 @@
 """Parity of the packed-row rel-pos kernel (attn_relpos_rows.hip, f16 / bf16 grids of any width at hd 64 and
 80) with the CPU oracle, on an MI355X, at the sizes where its tiling can go wrong."""
+import numpy as np
 import pytest
 import torch
 
@@ -74,3 +75,29 @@ def test_narrow_grids_read_nothing_past_a_head(hip, h, w, bh, hd, dtype):  # noq
     rest = [b for b in range(bh) if b != 1]
     assert (got[rest] == clean[rest]).all()
     assert torch.from_numpy(got[1]).isnan().all()
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("h,w,rows", [(11, 33, (6, 8)), (11, 33, (0, 2)), (9, 13, (0, 4)), (51, 3, (26, 34))])
+def test_tiles_of_infinite_keys(hip, h, w, rows, hd, dtype):  # noqa: F811
+    """Infinite keys that fill the first tile of a wave group (the second's, the first's, a lone one's) give a
+    query scores of -inf, weight 0, or of +inf, a NaN row, by the sign of its q."""
+    bh, dim = 2, 5
+    print(f"infinite keys {dtype} {h}x{w} rows {rows} hd={hd}", flush=True)
+    q, kt, v, table = make_inputs(h, w, bh, hd, 8, dtype)
+    keys = slice(rows[0] * w, rows[1] * w)
+    kt[0, dim, keys] = np.inf
+    got = run_gpu(hip, [q, kt, v, table], h, w, hd ** -0.5, dtype)
+    masked = q[0, :, dim] < 0
+    assert masked.any() and not masked.all()
+    assert np.isnan(got[0][~masked]).all()
+    kt[0, dim, keys] = 0
+    i, j = np.divmod(np.arange(h * w), w)
+    q64, t = q[0].astype(np.float64), table.astype(np.float64)
+    bias = np.einsum("nd,nkd->nk", q64, t[i[:, None] - i[None] + h - 1] + t[2 * h - 1 + j[:, None] - j[None] + w - 1])
+    logits = q64 @ kt[0].astype(np.float64) * hd ** -0.5 + bias
+    logits[:, keys] = -np.inf
+    p = np.exp(logits - logits.max(1, keepdims=True))
+    want = (p / p.sum(1, keepdims=True)) @ v[0].astype(np.float64)
+    check(got[0][masked], want[masked].astype(np.float32), dtype, f"infinite keys {h}x{w} hd={hd} {dtype}")
