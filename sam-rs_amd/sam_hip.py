@@ -119,10 +119,17 @@ def enabled() -> bool:
     return bool(load().sam_hip_enabled())
 
 
+# torch's own accessors of the current device and its stream's handle; a torch without them takes the public call
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream():
     # the handle alone: torch.cuda.current_stream() looks the device up and builds a Stream around it, which
     # took 3 us of the 12.1 that a deform_core call takes the host (9.3 without)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is None or _raw_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_raw_device())
 
 
 def _ptr(t):
