@@ -12,10 +12,10 @@ constexpr int gcd8(int c) { return c % 8 == 0 ? 8 : (c % 4 == 0 ? 4 : (c % 2 == 
 constexpr int period(int cpr) { return cpr / gcd8(cpr); }  // tiles after which the chunk pattern repeats
 
 // The last chunk of a row from this one on reaches past the head's end in the last hd row: row W + 8 CPR > H W.
-// It is the last row but for widths below 4, where the 8 columns of a chunk span several rows.
+// It is the last row but for widths below 4, where the 8 columns of a chunk span several rows: H + 1 - ceil(8 / W)
+// there (no division: its result would sit in a vector register).
 constexpr int first_end_row(int H, int W, int cpr) {
-  const int r = H + 1 - (8 * cpr + W - 1) / W;
-  return r < H - 1 ? r : H - 1;
+  return H - (cpr > 1 || W > 3 ? 1 : W == 3 ? 2 : W == 2 ? 3 : 7);
 }
 // whether tile t holds a chunk of a row from `first` on
 constexpr bool reaches_row(int t, int r0, int first, int cpr) { return 8 * t + 8 > (first - r0) * cpr; }
