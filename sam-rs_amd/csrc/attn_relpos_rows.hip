@@ -250,7 +250,9 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
   const T* vl = vbase + (4 * (g4 >> 1) + (gi >> 2)) * kVStride + 16 * (g4 & 1) + 4 * (gi & 3);
 
   const float sc = scale * kLog2e;
-  float m_run = -INFINITY, l_run = 0.f;
+  // The maximum starts at a finite value: infinite keys can make all of a query's scores in a group's tiles so far
+  // -inf, and those must weigh 0. (A test for it in the loop takes a register and two instructions a tile.)
+  float m_run = -3e38f, l_run = 0.f;
   f32x16 o[kMBO];
 #pragma unroll
   for (int ob = 0; ob < kMBO; ++ob) o[ob] = f32x16{};
@@ -302,20 +304,18 @@ __global__ __launch_bounds__(NWV * 64, 2) void attn_relpos_rows_kernel(
       const float mt = max_with_partner32(mm * sc);
       if (wave_any(mt > m_run + kSlack)) {
         const float m_new = fmaxf(m_run, mt);
-        const float alpha = m_run == -INFINITY ? 0.f : exp2_fast(m_run - m_new);
+        const float alpha = exp2_fast(m_run - m_new);
         l_run *= alpha;
 #pragma unroll
         for (int ob = 0; ob < kMBO; ++ob) o[ob] *= alpha;
         m_run = m_new;
       }
-      // infinite keys: all of a query's scores in a group's tiles so far can be -inf (weight 0)
-      const float c = m_run == -INFINITY ? 0.f : -m_run;
       X8 b[4], blo[4];
 #pragma unroll
       for (int w4 = 0; w4 < 4; ++w4) {
         float pv[8];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) pv[e] = exp2_fast(fmaf(s_cur[w4 >> 1][8 * (w4 & 1) + e], sc, c));
+        for (int e = 0; e < 8; ++e) pv[e] = exp2_fast(fmaf(s_cur[w4 >> 1][8 * (w4 & 1) + e], sc, -m_run));
         if constexpr (kSplitP)
           split_hi_lo(pv, b[w4], blo[w4]);
         else
