@@ -483,17 +483,22 @@ static hipError_t pick_cpr(const void* q, const void* kt, const void* v, const v
 // divided by the scale, as in the 64-column kernel); returns false (nothing launched) for other shapes.
 // Widths of 25..32 and 57..64 pack no better than the general kernel's tiles of two or one whole rows. Its
 // steps are a little shorter there when the width is even, so it keeps what is not split, except at hd 64
-// past one round of workgroups (f16, this kernel against it: 16 heads of 60 x 60 at hd 80 107 / 103 us, 32
-// of 64 x 32 at hd 64 57.3 / 53.7, 300 of 24 x 32 at hd 64 85.4 / 105; odd widths gain, bf16 59 x 63 132 /
-// 214).
+// past one round of workgroups (bf16, this kernel against it: 43 heads of 33 x 58 131 / 135 us, 60 of 60 x 58
+// 448 / 459), and in f16 only where two of this kernel's workgroups share a CU, their registers (25..32 columns)
+// and their bias scratch of max(h, w) rows both fitting: 273 heads of 27 x 32 115 / 142, 152 of 32 x 26 78 / 96, but
+// 146 of 52 x 32 196 / 182, and of one workgroup a CU 69 of 56 x 62 382 / 368. Odd widths gain (bf16 59 x 63
+// 132 / 214).
 bool attn_relpos_rows(int dtype, const void* q, const void* kt, const void* v, const void* table, void* out, int bh,
                       int hd, int h, int w, float scale, hipStream_t stream, hipError_t* err) {
   const float sc = scale * kLog2e;
   if ((hd != 80 && hd != 64) || h < 1 || h > 64 || w < 1 || w > 64 || !(sc >= 0.015625f && sc <= 4.f)) return false;
   const int cpr = (w + 7) / 8;
-  if ((cpr == 4 || cpr == 8) && w % 2 == 0 && h * w > 128 && !rows_split(bh, h, w) &&
-      (hd == 80 || (long)bh * ((h * w + 255) / 256) <= device_cu_count()))
-    return false;
+  if ((cpr == 4 || cpr == 8) && w % 2 == 0 && h * w > 128 && !rows_split(bh, h, w)) {
+    const bool one_round = (long)bh * ((h * w + 255) / 256) <= device_cu_count();
+    const size_t lds = rows::Shape<64>::kTiles * sizeof(f16) + (size_t)8 * ((h > w ? h : w) + 1) * 32 * sizeof(float);
+    const bool two_a_cu = cpr == 4 && 2 * lds <= 160 * 1024;
+    if (hd == 80 || one_round || (dtype == kF16 && !two_a_cu)) return false;
+  }
   if (hd == 80)
     *err = dtype == kF16 ? pick_cpr<f16, 80>(q, kt, v, table, out, bh, h, w, scale, stream)
                          : pick_cpr<bf16, 80>(q, kt, v, table, out, bh, h, w, scale, stream);

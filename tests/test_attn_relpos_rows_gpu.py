@@ -101,3 +101,16 @@ def test_tiles_of_infinite_keys(hip, h, w, rows, hd, dtype):  # noqa: F811
     p = np.exp(logits - logits.max(1, keepdims=True))
     want = (p / p.sum(1, keepdims=True)) @ v[0].astype(np.float64)
     check(got[0][masked], want[masked].astype(np.float32), dtype, f"infinite keys {h}x{w} hd={hd} {dtype}")
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+@pytest.mark.parametrize("h,w,bh", [(10, 26, 140), (39, 32, 60), (40, 32, 60), (9, 60, 90)])
+def test_even_widths_past_a_round(hip, h, w, bh, dtype):  # noqa: F811
+    """Even widths of 25..32 and 57..64 at hd 64 past one round of workgroups, on both sides of the line between
+    this kernel and the general one (39 rows are the last whose scratch lets two workgroups share a CU)."""
+    print(f"even widths {dtype} {h}x{w} bh={bh}", flush=True)
+    q, kt, v, table = make_inputs(h, w, bh, 64, 60 + h, dtype, table_std=0.5)
+    got = run_gpu(hip, [q, kt, v, table], h, w, 0.125, dtype)
+    heads = [0, bh // 2, bh - 1]
+    want = oracle.attention_relpos(q[heads], kt[heads], v[heads], table, h, w, 0.125)
+    check(got[heads], want, dtype, f"even widths {h}x{w} {dtype}")
