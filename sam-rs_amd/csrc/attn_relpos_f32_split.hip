@@ -17,8 +17,8 @@
 //   * a tile's products and weights are summed by themselves and then added to the running ones, so the
 //     rounding of a long row grows with its tiles, not with its keys.
 //   * G = 2: two groups of waves take half of the grid rows each for the same queries and merge at the end.
-// An infinity splits into inf - inf, so a row whose result is not finite is computed again in plain f32
-// (relpos_f32_row): infinities and NaN come out as f32 arithmetic has them.
+// An infinity splits into inf - inf, so a row whose result is not finite is computed again on the f32 matrix
+// units (relpos_f32_rows): infinities and NaN come out as f32 arithmetic has them.
 #include <type_traits>
 
 #include "common.hpp"
@@ -37,6 +37,9 @@ template <int HD> struct Shape {
   static constexpr int kKPlane = HD * 32, kVPlane = 32 * kVS;
   static constexpr int kBuf = 3 * (kKPlane + kVPlane);  // elements of one tile
 };
+
+// 4-wave workgroups at hd 64 hold up to 5 chunks a row in 168 registers, so that three share a CU
+constexpr int waves_per_simd(int hd, int cpr, int qw, int g) { return hd == 64 && cpr <= 5 && qw * g == 4 ? 3 : 2; }
 
 constexpr int gcd4(int c) { return c % 4 == 0 ? 4 : (c % 2 == 0 ? 2 : 1); }
 constexpr int period(int cpr) { return cpr / gcd4(cpr); }  // tiles after which the chunk pattern repeats
@@ -84,44 +87,115 @@ __device__ __forceinline__ f32x16 mma6(const bf16x8* a, const bf16x8* b, f32x16 
 
 }  // namespace f32s
 
-// One output row in plain f32 by a whole wave: the maximum of the scores, then weights, their sum and the
-// weighted sum of v, 64 keys at a time. Only rows whose result is not finite come here.
+// The 32 queries of a wave (from q0, one a lane of either half) on the f32 matrix units, straight from memory:
+// 32 keys of one grid row a tile, logits (q . k) * scale + rh + rw, accurate expf. rhs is the wave's own bias
+// scratch, rows of 32. Only the rows in `bad` are stored. Nothing is staged: bound by the latency of its loads. With a
+// NaN in every head, 12 heads of 64 x 64 at hd 64 take 1.24 ms (0.33 clean; the f32 MFMA kernel before 0.6; one wave
+// a row in plain f32, as this was first done, 42), 300 windows of 14 x 14 0.19 (2.3).
 template <int HD>
-__device__ __forceinline__ void relpos_f32_row(const float* __restrict__ q, const float* __restrict__ kt,
-                                               const float* __restrict__ v, const float* __restrict__ table,
-                                               float* __restrict__ out, int qi, int qj, int H, int W, float scale) {
-  const int lane = threadIdx.x & 63, N = H * W;
-  auto score = [&](int k) {
-    const int kh = k / W, kw = k - kh * W;
-    const float* th = table + (long)(qi - kh + H - 1) * HD;
-    const float* tw = table + (long)(2 * H - 1 + qj - kw + W - 1) * HD;
-    float s = 0.f, rh = 0.f, rw = 0.f;
-    for (int d = 0; d < HD; ++d) {
-      s = fmaf(q[d], kt[(long)d * N + k], s);
-      rh = fmaf(q[d], th[d], rh);
-      rw = fmaf(q[d], tw[d], rw);
-    }
-    return s * scale + rh + rw;
+__device__ __forceinline__ void relpos_f32_rows(const float* __restrict__ q, const float* __restrict__ kt,
+                                                const float* __restrict__ v, const float* __restrict__ table,
+                                                float* __restrict__ out, float* rhs, int q0, unsigned bad, int H, int W,
+                                                float scale) {
+  constexpr int kHalf = HD / 2, kMBO = (HD + 31) / 32;  // k-step s takes dims s (lower lanes) and kHalf + s (upper)
+  constexpr float kSlackNat = 5.5451774f;               // 8 ln 2
+  const int lane = threadIdx.x & 63, n = lane & 31, hh = lane >> 5, N = H * W;
+  const int qidx = min(q0 + n, N - 1), qi = qidx / W, qj = qidx % W;
+  auto wsync = [&]() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   };
-  float m = -INFINITY;
-  for (int k = lane; k < N; k += 64) m = fmaxf(m, score(k));
-  for (int x = 32; x > 0; x >>= 1) m = fmaxf(m, __shfl_xor(m, x));
-  float l = 0.f, o0 = 0.f, o1 = 0.f;
-  for (int k0 = 0; k0 < N; k0 += 64) {
-    const int cnt = min(64, N - k0);
-    const float p = lane < cnt ? expf(score(k0 + lane) - m) : 0.f;
-    l += p;
-    for (int j = 0; j < cnt; ++j) {
-      const float pj = __shfl(p, j);
-      const float* vr = v + (long)(k0 + j) * HD;
-      o0 = fmaf(pj, vr[lane], o0);
-      if (HD > 64 && lane < HD - 64) o1 = fmaf(pj, vr[64 + lane], o1);
+  float qf[kHalf];
+#pragma unroll
+  for (int s = 0; s < kHalf; s += 4) {
+    const f32x4 x = *reinterpret_cast<const f32x4*>(q + (long)qidx * HD + kHalf * hh + s);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) qf[s + e] = x[e];
+  }
+  // rhs[k] = q . tab[base - k + len - 1]
+  auto band = [&](const float* tab, int base, int len) {
+    wsync();
+    for (int b = 0; b < 2 * len - 1; b += 32) {
+      const float* trow = tab + (long)min(b + n, 2 * len - 2) * HD + kHalf * hh;
+      f32x16 acc = {};
+#pragma unroll
+      for (int s = 0; s < kHalf; s += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(trow + s);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], qf[s + e], acc, 0, 0, 0);
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int k = base + len - 1 - b - (8 * (e >> 2) + 4 * hh + (e & 3));
+        if (k >= 0 && k < len) rhs[k * 32 + n] = acc[e];
+      }
+    }
+    wsync();
+  };
+  float m = -INFINITY, l = 0.f;
+  f32x16 o[kMBO];
+#pragma unroll
+  for (int ob = 0; ob < kMBO; ++ob) o[ob] = f32x16{};
+  for (int c0 = 0; c0 < W; c0 += 32) {
+    band(table + (long)(2 * H - 1) * HD, qj, W);
+    float rw[16];  // columns c0 + 8 (e / 4) + 4 hh + e % 4
+#pragma unroll
+    for (int e = 0; e < 16; ++e) rw[e] = rhs[min(c0 + 8 * (e >> 2) + 4 * hh + (e & 3), W - 1) * 32 + n];
+    band(table, qi, H);
+    for (int row = 0; row < H; ++row) {
+      unsigned col0 = c0 + 4 * hh;  // as the asm leaves it: what follows is computed here, not held for every row
+      asm volatile("" : "+v"(col0));
+      const float* kcol = kt + (long)kHalf * hh * N + row * W + min(c0 + n, W - 1);
+      f32x16 s = {};
+#pragma unroll
+      for (int d = 0; d < kHalf; ++d) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kcol[(long)d * N], qf[d], s, 0, 0, 0);
+      const float rh = rhs[row * 32 + n];
+      float mm = -INFINITY;
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const float x = s[e] * scale + rh + rw[e];
+        s[e] = (int)col0 + 8 * (e >> 2) + (e & 3) < W ? x : -INFINITY;
+        mm = fmaxf(mm, s[e]);
+      }
+      const float mt = max_with_partner32(mm);
+      if (wave_any(mt > m + kSlackNat)) {
+        const float m_new = fmaxf(m, mt);
+        const float alpha = m == -INFINITY ? 0.f : expf(m - m_new);
+        l *= alpha;
+#pragma unroll
+        for (int ob = 0; ob < kMBO; ++ob) o[ob] *= alpha;
+        m = m_new;
+      }
+      const float c = m == -INFINITY ? 0.f : m;  // all scores so far -inf: weight 0
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        s[e] = expf(s[e] - c);
+        l += s[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) {
+        const int col = (int)col0 + 8 * (e >> 2) + (e & 3);
+        const unsigned voff = (unsigned)((row * W + min(col, W - 1)) * HD);
+#pragma unroll
+        for (int ob = 0; ob < kMBO; ++ob) {
+          const float a = v[voff + (unsigned)min(32 * ob + n, HD - 1)];
+          o[ob] = __builtin_amdgcn_mfma_f32_32x32x2f32(col < W ? a : 0.f, s[e], o[ob], 0, 0, 0);
+        }
+      }
     }
   }
-  for (int x = 32; x > 0; x >>= 1) l += __shfl_xor(l, x);
-  const float inv = 1.f / l;
-  out[lane] = o0 * inv;
-  if (HD > 64 && lane < HD - 64) out[64 + lane] = o1 * inv;
+  const float inv = 1.f / sum_with_partner32(l);
+  if ((bad >> n) & 1) {
+    float* orow = out + (long)(q0 + n) * HD;
+#pragma unroll
+    for (int ob = 0; ob < kMBO; ++ob)
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+        if (32 * ob + 8 * a < HD)
+          *reinterpret_cast<f32x4*>(orow + 32 * ob + 8 * a + 4 * hh) =
+              f32x4{o[ob][4 * a] * inv, o[ob][4 * a + 1] * inv, o[ob][4 * a + 2] * inv, o[ob][4 * a + 3] * inv};
+  }
 }
 
 // QW waves of 32 queries in each of G groups; NB tile buffers a group (2: one barrier a tile; 1: two, for
@@ -129,7 +203,7 @@ __device__ __forceinline__ void relpos_f32_row(const float* __restrict__ q, cons
 // products in 334 us, 1.23 PFLOP/s, what a large bf16 GEMM reaches on the card (1.19). The f32 MFMA kernel
 // before it took 700 us (16 heads), 567 (12 heads, now 287), and 71 for 300 windows of 14 x 14 (now 38).
 template <int HD, int CPR, int QW, int G, int NB>
-__global__ __launch_bounds__(QW* G * 64, 2) void attn_relpos_f32_split_kernel(
+__global__ __launch_bounds__(QW* G * 64, f32s::waves_per_simd(HD, CPR, QW, G)) void attn_relpos_f32_split_kernel(
     const float* __restrict__ q, const float* __restrict__ kt, const float* __restrict__ v,
     const float* __restrict__ table, float* __restrict__ out, int H, int W, float scale, float sc, int qblocks) {
   using namespace f32s;
@@ -454,12 +528,12 @@ __global__ __launch_bounds__(QW* G * 64, 2) void attn_relpos_f32_split_kernel(
   }
   unsigned long bad = __builtin_amdgcn_ballot_w64(!finite);
   bad = (bad | (bad >> 32)) & 0xffffffffu;
-  while (bad) {  // the same address and wave as the store above, so later in order
-    const int r = q0 + __builtin_ctzl(bad);
-    bad &= bad - 1;
-    relpos_f32_row<HD>(q + (bh * N + r) * HD, kt + bh * HD * (long)N, v + bh * HD * (long)N, table,
-                       out + (bh * N + r) * HD, r / W, r % W, H, W, scale);
-  }
+  // The same wave as the stores above, so later in order; rhs is this wave's alone by now. Never expected: otherwise
+  // the compiler gives up registers of the key loop for it (109 heads of 29 x 16 at hd 80 58.7 us without these rows'
+  // code, 64.8 with it, 59.6 so).
+  if (__builtin_expect_with_probability(bad != 0, 0, 1.0))
+    relpos_f32_rows<HD>(q + bh * HD * (long)N, kt + bh * HD * (long)N, v + bh * HD * (long)N, table,
+                        out + bh * HD * (long)N, rhs, q0, (unsigned)bad, H, W, scale);
 }
 
 template <int HD, int CPR, int QW, int G, int NB>
