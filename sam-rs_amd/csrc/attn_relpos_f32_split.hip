@@ -17,8 +17,10 @@
 //   * a tile's products and weights are summed by themselves and then added to the running ones, so the
 //     rounding of a long row grows with its tiles, not with its keys.
 //   * G = 2: two groups of waves take half of the grid rows each for the same queries and merge at the end.
-// An infinity splits into inf - inf, so a row whose result is not finite is computed again on the f32 matrix
-// units (relpos_f32_rows): infinities and NaN come out as f32 arithmetic has them.
+// An infinity splits into inf - inf, and what a low term has below 2^-133 is lost (of values below 2^-110 some of
+// the 24 bits: v of about 2^-120 gave 9e-5 of relative error). So a row with a result that is not finite, or not 0
+// and below 2^-104, is computed again on the f32 matrix units (relpos_f32_rows): infinities, NaN and small values
+// come out as f32 arithmetic has them. In a score the loss is 2^-133 of the other factor.
 #include <type_traits>
 
 #include "common.hpp"
@@ -29,6 +31,8 @@ namespace samhip {
 namespace f32s {
 
 constexpr float kSlack = 8.0f;  // log2 units by which a weight may exceed 1 before the maximum moves
+// least result that the three terms hold in full: what they lose is below 2^-133, the last bit of a small bf16
+constexpr unsigned kLeastHeld = (127 - 104) << 23;  // 2^-104
 
 template <int HD> struct Shape {
   static constexpr int kKS = HD / 16;
@@ -49,7 +53,7 @@ __device__ __forceinline__ int xcd_block(int i, int total) {
   return x * per + (x < rem ? x : rem) + j;
 }
 
-// x = hi + mid + lo, exact for every finite x whose low term is a normal number. Two at a time on the packed
+// x = hi + mid + lo, exact for every finite x whose low term keeps its bits (|x| from 2^-110 on). Two at a time on the packed
 // conversion; the terms go back to f32 by a shift and a mask.
 struct Split {
   bf16x8 t[3];
@@ -508,7 +512,8 @@ __global__ __launch_bounds__(QW* G * 64, f32s::waves_per_simd(HD, CPR, QW, G)) v
 
   // ---- normalise and store: lane holds O^T[32*ob + 8*a + 4*hh + b][query n]
   const float inv = 1.f / l;
-  bool finite = true;
+  unsigned least = ~0u;  // of 2 |bits| - 1, which puts 0 last
+  float most = 0.f;
   if (qvalid) {
     float* orow = out + (bh * N + qidx) * HD;
 #pragma unroll
@@ -520,13 +525,14 @@ __global__ __launch_bounds__(QW* G * 64, f32s::waves_per_simd(HD, CPR, QW, G)) v
 #pragma unroll
           for (int b = 0; b < 4; ++b) {
             w4[b] = o[ob][4 * a + b] * inv;
-            finite = finite && __builtin_fabsf(w4[b]) < INFINITY;
+            least = min(least, 2 * __float_as_uint(w4[b]) - 1);
+            most = max_nc(most, __builtin_fabsf(w4[b]));
           }
           *reinterpret_cast<f32x4*>(orow + 32 * ob + 8 * a + 4 * hh) = w4;
         }
       }
   }
-  unsigned long bad = __builtin_amdgcn_ballot_w64(!finite);
+  unsigned long bad = __builtin_amdgcn_ballot_w64(least < 2 * kLeastHeld - 1 || !(most < INFINITY));
   bad = (bad | (bad >> 32)) & 0xffffffffu;
   // The same wave as the stores above, so later in order; rhs is this wave's alone by now. Never expected: otherwise
   // the compiler gives up registers of the key loop for it (109 heads of 29 x 16 at hd 80 58.7 us without these rows'

@@ -90,3 +90,28 @@ def test_rows_that_are_not_finite_are_not_slow(hip, h, w, bh, hd):  # noqa: F811
     assert out.isnan().all()
     print(f"clean {clean:.1f} us, not finite {bad:.1f} us", flush=True)
     assert bad <= 9 * clean
+
+
+@pytest.mark.parametrize("hd", [64, 80])
+@pytest.mark.parametrize("h,w,bh", [(9, 13, 3), (11, 33, 2)])
+@pytest.mark.parametrize("exponent", [-100, -112, -120])
+def test_small_values_keep_their_bits(hip, h, w, bh, hd, exponent):  # noqa: F811
+    """Values of v about 2^exponent, in every column and in one, lose nothing to the third bf16 term: the f32 bar
+    against 64 bits, relative to the column's largest result."""
+    print(f"small values {h}x{w} hd={hd} 2^{exponent}", flush=True)
+    q, kt, v, table = make_inputs(h, w, bh, hd, 31, "f32")
+    unit = np.ldexp(np.float32(1), exponent)
+    i, j = np.divmod(np.arange(h * w), w)
+    t = table.astype(np.float64)
+    rel = t[i[:, None] - i[None] + h - 1] + t[2 * h - 1 + j[:, None] - j[None] + w - 1]
+    for columns in (slice(None), slice(5, 6)):
+        small = v.copy()
+        small[:, :, columns] *= unit
+        got = run_gpu(hip, [q, kt, small, table], h, w, hd ** -0.5, "f32").astype(np.float64)
+        for b in range(bh):
+            qs = q[b].astype(np.float64)
+            s = qs @ kt[b].astype(np.float64) * hd ** -0.5 + np.einsum("nd,nkd->nk", qs, rel)
+            p = np.exp(s - s.max(1, keepdims=True))
+            want = (p / p.sum(1, keepdims=True)) @ small[b].astype(np.float64)
+            err = (np.abs(got[b] - want).max(0) / np.abs(want).max(0)).max()
+            assert err <= 1e-5, err
