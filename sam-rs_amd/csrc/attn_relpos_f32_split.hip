@@ -252,11 +252,14 @@ __global__ __launch_bounds__(QW* G * 64, f32s::waves_per_simd(HD, CPR, QW, G)) v
                                                        (int)(HD * N * sizeof(float)), 0x00020000);
   const auto vrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(v + bh * HD * (long)N), 0,
                                                        (int)(HD * N * sizeof(float)), 0x00020000);
-  // an odd remainder of items goes to the first waves for K and to the last ones for V
+  // At hd 80 the remainder of items goes to the first waves for K and to the last ones for V (16 heads of 37 x 50 132 us,
+  // 135 with both to the first). At hd 64, where 8 waves have half a round of each, the first four take both (12 heads
+  // of 64 x 64 282 us; 291 with V to the last four).
+  constexpr bool kFar = HD == 80 && kVItems % kGT != 0;
   auto kitem = [&](int u) { return gt + u * kGT; };
-  auto vitem = [&](int u) { return kVItems % kGT == 0 ? gt + u * kGT : kVItems - 1 - gt - u * kGT; };
+  auto vitem = [&](int u) { return (kFar ? kGT - 1 - gt : gt) + u * kGT; };
   auto kin = [&](int u) { return kKItems % kGT == 0 || u + 1 < KPT || kitem(u) < kKItems; };
-  auto vin = [&](int u) { return kVItems % kGT == 0 || u + 1 < VPT || vitem(u) >= 0; };
+  auto vin = [&](int u) { return kVItems % kGT == 0 || u + 1 < VPT || vitem(u) < kVItems; };
   auto load8 = [&](auto rsrc, int off, float* x) {
     const u32x4 a = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0);
     const u32x4 b = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off + 16, 0, 0);
