@@ -90,6 +90,9 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
   constexpr bool kSplitP = __is_same(T, bf16);
   // at 168 registers there is no room for V(t+1) beside the scores; the other two waves cover its latency
   constexpr bool kLateV = THREE && DP == 64;
+  // Past head dim 128 O and the scores leave no room for K(t+2) and V(t+1) at once (together they spilled up to
+  // 2000 registers): V's loads take K's place once K is stored, ahead of the P.V that hides them.
+  constexpr bool kMidV = DP > 128;
   constexpr int KS = FG::KS, MBO = FG::MBO, KSTR = FG::KSTR, VSTR = FG::VSTR;
   constexpr int KBUF = FG::KBUF, VBUF = FG::VBUF, NT = FG::NT;
   constexpr int CPR = FG::CPR, CH = FG::CH, PT = FG::PT;
@@ -111,7 +114,8 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
   const int d = p.d;
 
   const int q0 = qb * (NW * 32) + wave * 32;
-  const bool active = q0 < p.lq;
+  // a wave without queries only stages (past head dim 128, where a branch in the loop spills O, it computes on zeros)
+  const bool active = DP > 128 || q0 < p.lq;
   const int qidx = q0 + n;
   const bool qvalid = qidx < p.lq;
 
@@ -288,9 +292,24 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
   auto step = [&](int t, f32x16* s_cur, f32x16* s_nxt) {
     const int i = t - t_begin;
     load_k(min(t + 2, tl));
-    if (!kLateV) load_v(min(t + 1, tl));
+    if (!kLateV && !kMidV) load_v(min(t + 1, tl));
+    X8 b[4], blo[4];
+    auto pv_product = [&]() {
+      // O^T += V^T . P^T; in bf16, P is split into hi + lo bf16 terms so the product keeps ~16 bits of P
+      const T* vb = vs_base + (i & 1) * VBUF;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+#pragma unroll
+        for (int ob = 0; ob < MBO; ++ob) {
+          const T* p0 = vb + voff[u][0] + 32 * ob;
+          const T* p1 = vb + voff[u][1] + 32 * ob;
+          const X8 a = join8<T>(lds_read_tr16(p0), lds_read_tr16(p1));
+          o[ob] = mma32(a, b[u], o[ob]);
+          if (kSplitP) o[ob] = mma32(a, blo[u], o[ob]);
+        }
+      }
+    };
     if (active) {
-      X8 b[4], blo[4];
       float mv[2][16];
       if constexpr (MASK) load_mask(t, mv);
       // keys past the end of the last tile: -inf scores
@@ -350,29 +369,22 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
         }
       }
       l_run += lsum;
-      // O^T += V^T . P^T; in bf16, P is split into hi + lo bf16 terms so the product keeps ~16 bits of P
-      const T* vb = vs_base + (i & 1) * VBUF;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-#pragma unroll
-        for (int ob = 0; ob < MBO; ++ob) {
-          const T* p0 = vb + voff[u][0] + 32 * ob;
-          const T* p1 = vb + voff[u][1] + 32 * ob;
-          const X8 a = join8<T>(lds_read_tr16(p0), lds_read_tr16(p1));
-          o[ob] = mma32(a, b[u], o[ob]);
-          if (kSplitP) o[ob] = mma32(a, blo[u], o[ob]);
-        }
-      }
+      if constexpr (!kMidV) pv_product();
+    }
+    if constexpr (kMidV) {
+      store_k(i & 1);
+      load_v(min(t + 1, tl));
+      if (active) pv_product();
     }
     if (kLateV) load_v(min(t + 1, tl));
     // K(t+2) replaces K(t), whose scores were taken one step ago, V(t+1) replaces V(t-1)
-    store_k(i & 1);
+    if (!kMidV) store_k(i & 1);
     store_v(min(t + 1, tl), (i + 1) & 1);
     __syncthreads();
   };
 
   f32x16 sa[2], sb[2];
-  if (active) qk(ks_base, sa);  // a wave whose 32 queries are all past the end only stages
+  if (active) qk(ks_base, sa);
   __syncthreads();  // every wave has read K(0) before step 0 overwrites its buffer with K(2)
   for (int t = t_begin; t < t_end; t += 2) {
     step(t, sa, sb);
