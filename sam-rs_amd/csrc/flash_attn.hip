@@ -557,14 +557,16 @@ int flash_queries_per_block(int dtype, int d, int lk) {
 
 // Key splits, at least 2 key tiles per split. 4-wave f16 / bf16 workgroups (three resident per CU in
 // f16 up to head dim 64, two otherwise): the count that gives the least time among those that fit one round
-// of resident workgroups. A tile takes about 0.85 us (1.1 in bf16) alone on its CU and 0.6 times as much
+// of resident workgroups (a masked launch at head dim 33..64 runs two to a CU, so its plan takes no more splits
+// than the unmasked one that sizes the workspace). A tile takes about 0.85 us (1.1 in bf16) alone on its CU and 0.6 times as much
 // again for each workgroup beside it; merging costs about 3.3 us and 0.5 us per MB of partials. Measured
 // against as many splits as fit, in f16: 64 windows of 256 keys at head dim 72 18.2 -> 9.5 us (1 for 2), 4096 x 4096
 // over one head at 64 26.5 -> 18.5 (8 for 22), 8 heads of 1024 at 64 20.4 -> 14.9 (4 for 8); 12 heads of
 // 4096 keep 2, 13% faster than none, and one of 1024 at 72 its 8 (12.0 us, 16.2 with 2). Otherwise (8 waves,
 // f32, head dim 256): enough workgroups to give every CU its resident share (one workgroup per CU at head
 // dim 256, two below).
-void flash_plan(int dtype, int b, int h, int lq, int lk, int d, int cus, int* qblocks, int* nsplit, int* tps) {
+void flash_plan(int dtype, int b, int h, int lq, int lk, int d, bool masked, int cus, int* qblocks, int* nsplit,
+                int* tps) {
   const int qpb = flash_queries_per_block(dtype, d, lk);
   *qblocks = (lq + qpb - 1) / qpb;
   const int tiles = (lk + 63) / 64;
@@ -573,7 +575,7 @@ void flash_plan(int dtype, int b, int h, int lq, int lk, int d, int cus, int* qb
   const int maxs = tiles / 2 > 1 ? tiles / 2 : 1;
   int ns = 1;
   if (dtype != kF32 && dp <= 128 && qpb == 128) {
-    const long slots = (long)cus * (dtype == kF16 && dp <= 64 ? 3 : 2);
+    const long slots = (long)cus * (dtype == kF16 && dp <= (masked ? 32 : 64) ? 3 : 2);
     const float tile = dtype == kF16 ? 0.85f : 1.1f, mb = (float)b * h * lq * dp * 4e-6f;
     float best = INFINITY;
     for (int n = 1; n <= maxs && n <= 64 && (n == 1 || n * base <= slots); ++n) {

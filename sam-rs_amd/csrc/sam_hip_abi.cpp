@@ -381,12 +381,13 @@ size_t round256(size_t n) { return (n + 255) / 256 * 256; }
 
 // Workspace: key-split partials, then (when keys are rotated) the rotated keys and room for the rotated
 // queries, both contiguous [b, l, h, d], then (head dim 256) V as transposed key tiles.
+// A masked call's plan needs no more than the unmasked one, which the workspace queries give.
 // cu_cap > 0 plans as if the device had at most that many CUs (fewer key splits, a smaller workspace).
-FlashPlan plan_flash(int dtype, int b, int lq, int lk, int h, int d, int n_rope_k, int cu_cap) {
+FlashPlan plan_flash(int dtype, int b, int lq, int lk, int h, int d, int n_rope_k, bool masked, int cu_cap) {
   FlashPlan pl;
   int cus = device_cus();
   if (cu_cap > 0 && cus > cu_cap) cus = cu_cap;
-  samhip::flash_plan(dtype, b, h, lq, lk, d, cus, &pl.qblocks, &pl.nsplit, &pl.tps);
+  samhip::flash_plan(dtype, b, h, lq, lk, d, masked, cus, &pl.qblocks, &pl.nsplit, &pl.tps);
   pl.partial_bytes = round256(samhip::flash_partial_bytes(b, h, lq, d, pl.nsplit));
   const size_t elem = dtype == 0 ? 4 : 2;
   pl.krot_bytes = n_rope_k > 0 ? round256((size_t)b * lk * h * d * elem) : 0;
@@ -413,7 +414,7 @@ extern "C" {
 
 long sam_hip_flash_attn_workspace_size(int dtype, int b, int lq, int lk, int h, int d, int n_rope_k) {
   if (check_flash_sizes(dtype, b, lq, lk, h, d) != SAM_HIP_OK) return -1;
-  return (long)plan_flash(dtype, b, lq, lk, h, d, n_rope_k, 0).total;
+  return (long)plan_flash(dtype, b, lq, lk, h, d, n_rope_k, false, 0).total;
 }
 
 // sam_hip_flash_attn, and sam_hip_sdpa_mask when mask is not null (no RoPE then).
@@ -452,7 +453,7 @@ static int flash_entry(const void* q, const void* k, const void* v, void* out, i
       return fail(SAM_HIP_EUNSUPPORTED, "sdpa-mask: the mask must be aligned to its element size");
     p.mask = mask;
   }
-  const FlashPlan pl = plan_flash(dtype, b, lq, lk, h, d, n_rope_k, cu_cap);
+  const FlashPlan pl = plan_flash(dtype, b, lq, lk, h, d, n_rope_k, mask != nullptr, cu_cap);
   if (pl.total > 0 && (!workspace || workspace_bytes < (long)pl.total))
     return fail(SAM_HIP_EINVAL, "flash-attn: needs a workspace of %zu bytes (sam_hip_flash_attn_workspace_size), got %ld",
                 pl.total, workspace ? workspace_bytes : 0L);
@@ -547,7 +548,7 @@ namespace samhip {
 // most cu_cap CUs (sam_hip_flash_attn_noalloc, whose workspace has a fixed size).
 long flash_workspace_size_capped(int dtype, int b, int lq, int lk, int h, int d, int n_rope_k, int cu_cap) {
   if (check_flash_sizes(dtype, b, lq, lk, h, d) != SAM_HIP_OK) return -1;
-  return (long)plan_flash(dtype, b, lq, lk, h, d, n_rope_k, cu_cap).total;
+  return (long)plan_flash(dtype, b, lq, lk, h, d, n_rope_k, false, cu_cap).total;
 }
 int flash_attn_capped(const void* q, const void* k, const void* v, void* out, int dtype, int b, int lq, int lk, int h,
                       int d, const long* strides_q, const long* strides_k, const long* strides_v,

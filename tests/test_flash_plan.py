@@ -1,0 +1,45 @@
+"""The key-split plan of the flash-attention launches, on the CPU: the host function of the built library."""
+import ctypes
+import os
+
+import pytest
+
+import sam_hip
+
+DT = {"f32": 0, "f16": 1, "bf16": 2}
+CUS = 256
+
+
+@pytest.fixture(scope="module")
+def plan():
+    if not os.path.exists(sam_hip.LIB_PATH):
+        pytest.skip("libsam_hip.so is not built")
+    # samhip::flash_plan(int dtype, int b, int h, int lq, int lk, int d, bool masked, int cus, int*, int*, int*)
+    fn = ctypes.CDLL(sam_hip.LIB_PATH)._ZN6samhip10flash_planEiiiiiibiPiS0_S0_
+    fn.argtypes = [ctypes.c_int] * 6 + [ctypes.c_bool, ctypes.c_int] + [ctypes.POINTER(ctypes.c_int)] * 3
+    fn.restype = None
+
+    def call(dtype, h, lq, lk, d, masked=False):
+        out = [ctypes.c_int() for _ in range(3)]
+        fn(DT[dtype], 1, h, lq, lk, d, masked, CUS, *out)
+        return tuple(x.value for x in out)  # query blocks, splits, tiles per split
+
+    return call
+
+
+SIZES = [(h, lq, lk) for h in (1, 3, 13, 24, 60, 200) for lq in (17, 300, 1195, 4096) for lk in (64, 400, 1195, 4096)]
+
+
+@pytest.mark.parametrize("dtype", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("d", [32, 48, 64, 72, 128, 192, 256])
+def test_masked_plan_fits_the_workgroups_that_share_a_cu(plan, dtype, d):
+    """A masked launch at padded head dim 64 runs two workgroups to a CU in f16, three without a mask: its splits
+    stay within that, and within the workspace of the unmasked plan, which is what the size query gives."""
+    for h, lq, lk in SIZES:
+        blocks, plain, _ = plan(dtype, h, lq, lk, d)
+        masked_blocks, masked, _ = plan(dtype, h, lq, lk, d, masked=True)
+        assert masked_blocks == blocks and masked <= plain, (h, lq, lk)
+        if dtype == "f16" and d in (48, 64):
+            assert masked == 1 or masked * h * blocks <= 2 * CUS, (h, lq, lk)
+        else:
+            assert masked == plain, (h, lq, lk)
