@@ -555,14 +555,22 @@ int flash_queries_per_block(int dtype, int d, int lk) {
   return 32 * (dp <= 64 ? 4 : dp <= 128 ? (lk <= 16 * 64 ? 4 : 8) : 4);
 }
 
+// us of a 64-key tile of a 4-wave f16 / bf16 workgroup alone on its CU, by padded head dim (the slope of 6 to 16
+// tiles; one price of 0.85 / 1.1 for all had 32 heads of 128 x 512 at 128 in bf16 take one split, 24.0 us, where four
+// take 18.3, and 2 heads of 332 x 332 at 96 in f16 one, 12.3, where three take 10.8)
+static float flash_tile_us(int dtype, int dp) {
+  if (dtype == kF16) return dp <= 32 ? 0.77f : dp <= 64 ? 0.84f : dp <= 96 ? 0.92f : 1.32f;
+  return dp <= 32 ? 0.84f : dp <= 64 ? 1.05f : dp <= 96 ? 1.14f : 2.0f;
+}
+
 // Key splits, at least 2 key tiles per split. 4-wave f16 / bf16 workgroups (three resident per CU in
 // f16 up to head dim 64, two otherwise): the count that gives the least time among those that fit one round
 // of resident workgroups (a masked launch at head dim 33..64 runs two to a CU, so its plan takes no more splits
-// than the unmasked one that sizes the workspace). A tile takes about 0.85 us (1.1 in bf16) alone on its CU and 0.6 times as much
-// again for each workgroup beside it; merging costs about 3.3 us and 0.5 us per MB of partials. Measured
-// against as many splits as fit, in f16: 64 windows of 256 keys at head dim 72 18.2 -> 9.5 us (1 for 2), 4096 x 4096
-// over one head at 64 26.5 -> 18.5 (8 for 22), 8 heads of 1024 at 64 20.4 -> 14.9 (4 for 8); 12 heads of
-// 4096 keep 2, 13% faster than none, and one of 1024 at 72 its 8 (12.0 us, 16.2 with 2). Otherwise (8 waves,
+// than the unmasked one that sizes the workspace). A tile alone on its CU takes flash_tile_us and 0.6 times as much
+// again for each workgroup beside it; merging costs about 2.3 us and 0.5 us per MB of partials. Measured in f16
+// over 1 to 16 splits: 64 heads of 100 x 256 at head dim 64 1 (8.3 us, 10.3 with 2), one of 4096 x 4096 8 (19.9; 24.8
+// with 16), 8 of 1024 x 1024 4 (15.9; 20.3 with 8), 12 of 4096 x 4096 2 (78.1; 82.5 with 1), one of 1024 at 72 8 (11.6;
+// 15.8 with 2). Otherwise (8 waves,
 // f32, head dim 256): enough workgroups to give every CU its resident share (one workgroup per CU at head
 // dim 256, two below).
 void flash_plan(int dtype, int b, int h, int lq, int lk, int d, bool masked, int cus, int* qblocks, int* nsplit,
@@ -576,11 +584,11 @@ void flash_plan(int dtype, int b, int h, int lq, int lk, int d, bool masked, int
   int ns = 1;
   if (dtype != kF32 && dp <= 128 && qpb == 128) {
     const long slots = (long)cus * (dtype == kF16 && dp <= (masked ? 32 : 64) ? 3 : 2);
-    const float tile = dtype == kF16 ? 0.85f : 1.1f, mb = (float)b * h * lq * dp * 4e-6f;
+    const float tile = flash_tile_us(dtype, dp), mb = (float)b * h * lq * dp * 4e-6f;
     float best = INFINITY;
     for (int n = 1; n <= maxs && n <= 64 && (n == 1 || n * base <= slots); ++n) {
       const long beside = (n * base + cus - 1) / cus - 1;
-      const float time = tile * (1.f + 0.6f * beside) * ((tiles + n - 1) / n) + (n > 1 ? 3.3f + 0.5f * mb * n : 0.f);
+      const float time = tile * (1.f + 0.6f * beside) * ((tiles + n - 1) / n) + (n > 1 ? 2.3f + 0.5f * mb * n : 0.f);
       if (time < best) {
         best = time;
         ns = n;
