@@ -82,12 +82,16 @@ def test_head_dim_192_is_not_slow(hip, dtype):
     assert padded <= 3 * own
 
 
+@pytest.mark.parametrize("stride", [(1 << 24) - 8, 1 << 24, (1 << 26) + (1 << 21) + 8])
 @pytest.mark.parametrize("d", [64, 72])
-def test_row_strides_past_32_bits(hip, d):
-    """A row stride of 2^24 elements and more: the offsets of a tile no longer fit in 32 bits."""
-    n, stride = 3, (1 << 24) + 8
+def test_row_strides_past_32_bits(hip, d, stride):
+    """Row strides on both sides of 2^24 elements, from which on a whole tile's offsets are formed in 64 bits, and
+    one whose 63 rows do not fit in 32 (63 (2^26 + 2^21 + 8) > 2^32). 66 keys: a whole tile and a rest."""
+    n = 66
+    print(f"flash strides d={d} {stride}", flush=True)
     q = rn(1, "f16", 1, 20, 1, d)
-    k, v = (torch.empty_strided((1, n, 1, d), (0, stride, d, 1), device="cuda", dtype=torch.float16) for _ in "kv")
+    rows = torch.empty(n * stride, device="cuda", dtype=torch.float16)  # k at the start of a row, v behind it
+    k, v = (rows.as_strided((1, n, 1, d), (0, stride, d, 1), off) for off in (0, d))
     k.copy_(rn(2, "f16", 1, n, 1, d))
     v.copy_(rn(3, "f16", 1, n, 1, d))
     want = exact(*(x.transpose(1, 2) for x in (q, k, v))).transpose(1, 2)
