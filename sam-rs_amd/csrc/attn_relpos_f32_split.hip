@@ -14,8 +14,8 @@
 //   * K planes [hd][32 slots], 64-byte rows, and V planes [32 slots][hd]: four consecutive rows of 32 elements
 //     fall on all 64 banks (hd 64: the 32-column halves of rows 2, 3 mod 4 are swapped for that).
 //   * the softmax runs in the exp2 domain: u = s * (scale log2e) + (rh - m) + rw, one fma and one add a score.
-//   * a tile's products and weights are summed by themselves and then added to the running ones, so the
-//     rounding of a long row grows with its tiles, not with its keys.
+//   * a tile's weights are summed by themselves and then added to the running sum, so the rounding of a long
+//     row's denominator grows with its tiles; the products go straight into the running O.
 //   * G = 2: two groups of waves take half of the grid rows each for the same queries and merge at the end.
 // An infinity splits into inf - inf, and what a low term has below 2^-133 is lost (of values below 2^-110 some of
 // the 24 bits: v of about 2^-120 gave 9e-5 of relative error). So a row with a result that is not finite, or not 0
@@ -53,8 +53,8 @@ __device__ __forceinline__ int xcd_block(int i, int total) {
   return x * per + (x < rem ? x : rem) + j;
 }
 
-// x = hi + mid + lo, exact for every finite x whose low term keeps its bits (|x| from 2^-110 on). Two at a time on the packed
-// conversion; the terms go back to f32 by a shift and a mask.
+// x = hi + mid + lo, exact for every finite x whose low term keeps its bits (|x| from 2^-110 on). Two at a time on
+// the packed conversion; the terms go back to f32 by a shift and a mask.
 struct Split {
   bf16x8 t[3];
 };
@@ -79,7 +79,7 @@ __device__ __forceinline__ Split split3(const float* x) {
   return s;
 }
 
-// acc += a . b over the six products that f32 holds, the small ones first
+// acc += a . b over the six products that f32 holds; the small ones first, which helps where acc starts small (S^T)
 __device__ __forceinline__ f32x16 mma6(const bf16x8* a, const bf16x8* b, f32x16 acc) {
   acc = mma32(a[2], b[0], acc);
   acc = mma32(a[0], b[2], acc);
@@ -205,7 +205,7 @@ __device__ __forceinline__ void relpos_f32_rows(const float* __restrict__ q, con
 // QW waves of 32 queries in each of G groups; NB tile buffers a group (2: one barrier a tile; 1: two, for
 // workgroups that share a CU). Bound by the matrix units: 16 heads of 64 x 64 at hd 64 are 412 GFLOP of bf16
 // products in 334 us, 1.23 PFLOP/s, what a large bf16 GEMM reaches on the card (1.19). The f32 MFMA kernel
-// before it took 700 us (16 heads), 567 (12 heads, now 287), and 71 for 300 windows of 14 x 14 (now 38).
+// before it took 695 us (16 heads), 530 (12 heads, now 281), and 67 for 300 windows of 14 x 14 (now 37).
 template <int HD, int CPR, int QW, int G, int NB>
 __global__ __launch_bounds__(QW* G * 64, f32s::waves_per_simd(HD, CPR, QW, G)) void attn_relpos_f32_split_kernel(
     const float* __restrict__ q, const float* __restrict__ kt, const float* __restrict__ v,
@@ -569,9 +569,10 @@ static hipError_t launch_f32_split(const void* q, const void* kt, const void* v,
 // waves that take half of the keys each, or 256 queries on 8 waves. The time is that of the fullest CU, in us
 // at hd 64 as measured: a tile of 32 slots takes a SIMD's two waves 2.8 when every 4 waves stage their own
 // keys, 2.6 when 8 share them, and a wave that has its SIMD to itself 2.0; a round costs about 5 beside its
-// tiles. Measured (4 waves / two groups / 8 waves): 300 heads of 14 x 14 38 / 54 / 47, 12 of 64 x 64
-// 329 / 330 / 287, 24 of 33 x 37 90 / 70 / 100, 96 of 12 x 12 16.9 / 14.9 / 19.0; at hd 80 16 of 37 x 50
-// 174 / 130 / 196, 96 of 30 x 30 199 / 182 / 202, 16 of 48 x 56 295 / 305 / 258.
+// tiles. (The kernel has become 10-20% faster than these since they were fitted, in all three forms.) Measured
+// (4 waves / two groups / 8 waves): 300 heads of 14 x 14 37 / 53 / 48, 12 of 64 x 64 328 / 333 / 281, 24 of 33 x 37
+// 92 / 70 / 104, 96 of 12 x 12 18.2 / 16.5 / 20.2; at hd 80 16 of 37 x 50 186 / 141 / 207, 96 of 30 x 30
+// 187 / 188 / 202, 16 of 48 x 56 302 / 315 / 262.
 template <int HD, int CPR>
 static hipError_t f32_split_waves(const void* q, const void* kt, const void* v, const void* table, void* out, int bh,
                                   int h, int w, float scale, hipStream_t stream) {

@@ -129,10 +129,11 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
   const T* vbase = reinterpret_cast<const T*>(p.v) + bi * p.sv[0] + head * p.sv[2];
 
   // ---- K/V tile staging: global -> registers -> LDS, 16-byte chunks of the 64 x DP tile (loads of those
-  // past d read the row's last one and are not stored). A thread's chunks are the same (row, columns) in every tile, at 32-bit offsets from the
-  // tile's first row; where a round of threads covers whole rows (kStep) its next round is at a uniform
-  // distance. The last tile's rows past the end read the last key instead: its scores are masked, its V is
-  // stored as zeros. Row strides whose offsets do not fit in 32 bits take the path of the last tile.
+  // past d read the row's last one and are not stored). A thread's chunks are the same (row, columns) in every
+  // tile, at 32-bit offsets from the tile's first row; where a round of threads covers whole rows (kStep) its next
+  // round is at a uniform distance. The last tile's rows past the end read the last key instead: its scores are
+  // masked, its V is stored as zeros. Row strides of 2^24 elements and more (63 of which stay far inside 32 bits)
+  // take the path of the last tile, whose offsets have 64.
   constexpr bool kStep = NT % CPR == 0;
   constexpr int RS = NT / CPR;  // rows of a round
   const bool wide = max(p.sk[1], p.sv[1]) >= 1L << 24;

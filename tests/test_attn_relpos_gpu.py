@@ -281,9 +281,8 @@ def test_vit_b_f32_layers(hip):
 
 
 def test_vit_l_f32_global_layer(hip):
-    """ViT-L f32 global layer (16 x 64x64, hd 64): its 1024 workgroups of 64 queries would take 1.33
-    rounds of the 16-queries-per-wave kernel, so it runs on the 32-queries-per-wave kernel; the oracle
-    checks heads 0, 8 and 15."""
+    """ViT-L f32 global layer (16 x 64x64, hd 64), one round of 256 workgroups of 256 queries on the kernel of
+    three bf16 terms; the oracle checks heads 0, 8 and 15."""
     print("vit-l f32 global", flush=True)
     arrays = make_inputs(64, 64, 16, 64, 12, "f32", qkv_std=0.55)
     got = run_gpu(hip, arrays, 64, 64, 0.125, "f32")
