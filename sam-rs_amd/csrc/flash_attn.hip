@@ -93,11 +93,6 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
   // Past head dim 128 O and the scores leave no room for K(t+2) and V(t+1) at once (together they spilled up to
   // 2000 registers): V's loads take K's place once K is stored, ahead of the P.V that hides them.
   constexpr bool kMidV = DP > 128;
-  // Nothing is fetched or stored past the last tile where that pays: 4 waves at 65..80 and 97..128, whose key ranges
-  // are short (bf16, 70 x 70 at 128 10.1 -> 9.0 us, 5 heads of 113 x 39 at 72 7.1 -> 6.5; 64 x 4 windows of 196 at 72
-  // 16.6 -> 15.9). Elsewhere the test costs more than the fetches: f16, 16 heads of 1024 at 96 23.2 -> 24.8, 12 of
-  // 4096 at 32 59.7 -> 62.0, 8 of 2000 at 200 67.7 -> 94.1, and masked 150 heads of 196 at 72 15.5 -> 17.1.
-  constexpr bool kStop = !MASK && NW == 4 && (DP == 80 || DP == 128);
   constexpr int KS = FG::KS, MBO = FG::MBO, KSTR = FG::KSTR, VSTR = FG::VSTR;
   constexpr int KBUF = FG::KBUF, VBUF = FG::VBUF, NT = FG::NT;
   constexpr int CPR = FG::CPR, CH = FG::CH, PT = FG::PT;
@@ -294,12 +289,11 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
   };
 
   // Softmax and P.V of tile t (scores in s_cur, buffers t&1) with the S^T of tile t+1 into s_nxt.
-  // Past the last tile the loads (unless kStop) and the next S^T run on clamped indices and their results go unused.
+  // Past the last tile the loads and the next S^T run on clamped indices and their results go unused.
   auto step = [&](int t, f32x16* s_cur, f32x16* s_nxt) {
     const int i = t - t_begin;
-    const bool more_k = !kStop || t + 2 <= tl, more_v = !kStop || t + 1 <= tl;
-    if (more_k) load_k(min(t + 2, tl));
-    if (!kLateV && !kMidV && more_v) load_v(min(t + 1, tl));
+    load_k(min(t + 2, tl));
+    if (!kLateV && !kMidV) load_v(min(t + 1, tl));
     X8 b[4], blo[4];
     auto pv_product = [&]() {
       // O^T += V^T . P^T; in bf16, P is split into hi + lo bf16 terms so the product keeps ~16 bits of P
@@ -385,8 +379,8 @@ __global__ __launch_bounds__(NW * 64, (THREE ? 3 : DP <= 128 ? 2 : 1)) void flas
     }
     if (kLateV) load_v(min(t + 1, tl));
     // K(t+2) replaces K(t), whose scores were taken one step ago, V(t+1) replaces V(t-1)
-    if (!kMidV && more_k) store_k(i & 1);
-    if (more_v) store_v(min(t + 1, tl), (i + 1) & 1);
+    if (!kMidV) store_k(i & 1);
+    store_v(min(t + 1, tl), (i + 1) & 1);
     __syncthreads();
   };
 
