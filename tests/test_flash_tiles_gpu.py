@@ -61,8 +61,8 @@ def test_head_dims_past_128(hip, d, lq, lk, dtype):
 
 @pytest.mark.parametrize("dtype", ["f16", "bf16"])
 def test_head_dim_192_is_not_slow(hip, dtype):
-    """Head dim 192 costs what the padded 256 does: 1.4 times head dim 256 on its own kernel as measured, 3 here (it
-    was 14 with its registers spilled in the key loop)."""
+    """Head dim 192 costs what the padded 256 does: 1.2 times head dim 256 on its own kernel as measured, 3 here (it
+    was 6.8 with its registers spilled in the key loop)."""
 
     def us(d):
         q, k, v = (rn(i, dtype, 1, 600, 24, d) for i in (1, 2, 3))
